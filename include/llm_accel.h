@@ -358,7 +358,9 @@ typedef struct {
                                          last (the generated forwards and their
                                          argmaxes) */
     /* Residency (tests/test_coarse_task_residency_contract.sh:63-80 of the
-     * reference): host -> device copies of hidden rows (one per forward),
+     * reference): host -> device moves of hidden rows (one per block of
+     * prompt rows and per generated forward; the blocks of a prompt that
+     * runs layer by layer travel in one copy),
      * device -> host copies of hidden rows (0: the argmax runs on the
      * device and returns 8-byte keys), KV transfers (0), key read-backs
      * (one per sampled token). */
@@ -387,6 +389,10 @@ int llm_set_log(llm_ctx_t* ctx, llm_log_fn fn, void* user);
  * (Tasks 18/19 per layer and 20) for every sampled token but the last.
  * Embedding rows are gathered on the host from `embedding` [vocab][hidden]
  * and uploaded, as in the reference.  Requires llm_load_lm_head first.
+ * A prompt of several blocks runs layer by layer over many rows at once
+ * (no line sink set, hidden >= 128): every row's values, the K/V cache, the
+ * hidden pairs and the counts are those of the block by block loop, and
+ * prompt_forward_ms is the time of the whole.
  * A one-launch kernel whose bounded wait between workgroups gives up
  * (e.g. a device shared with other work) does not fail the request: the
  * forwards since the previous synchronisation run again on launches

@@ -27,6 +27,7 @@
 #include "fixed_point.h"
 #include "kernels.h"
 #include "ops.h"
+#include "prefill.h"
 
 namespace {
 
@@ -254,6 +255,22 @@ struct llm_ctx {
     std::vector<hipEvent_t> gen_events;
     llm_log_fn log_fn = nullptr;
     void* log_user = nullptr;
+    // Layer-major prompt path (prefill.h) of llm_generate: its buffers, one
+    // allocation sized for `rows` rows (a multiple of kPfRowPad), made by the
+    // first prompt that takes it and replaced by a larger one when a longer
+    // prompt comes; LLM_ACCEL_PROMPT=0 keeps the prompt in blocks
+    struct Prompt {
+        uint32_t rows = 0;
+        uint8_t* base = nullptr;
+        int16_t *in = nullptr, *ha = nullptr, *hb = nullptr, *qkv = nullptr;
+        int8_t *xn = nullptr, *xa = nullptr, *act = nullptr, *qp = nullptr, *kp = nullptr,
+               *vp = nullptr;
+        int32_t *kbias = nullptr, *rowsum = nullptr;
+        uint32_t *kvflag = nullptr, *qflag = nullptr, *count = nullptr;
+        int64_t* part = nullptr;
+        size_t part_bytes = 0;
+    } pf;
+    bool prompt_path = true;
     uint64_t n_h2d_rows = 0;   // hidden-row uploads (calls)
     uint64_t n_d2h_rows = 0;   // hidden-row downloads (calls)
     uint64_t n_kv_moves = 0;   // KV reads / writes (calls)
@@ -1200,6 +1217,8 @@ int llm_ctx_create(const llm_shape_t* shape, int device, uint32_t num_pairs,
         return cleanup(fail(LLM_E_NOMEM, "hipHostMalloc failed"));
     *c->host_abort = 0;
     if (const char* e = std::getenv("LLM_ACCEL_FUSED")) c->fused = std::strcmp(e, "0") != 0;
+    if (const char* e = std::getenv("LLM_ACCEL_PROMPT"))
+        c->prompt_path = std::strcmp(e, "0") != 0;
     if (const char* e = std::getenv("LLM_ACCEL_GQA")) c->gqa = std::strcmp(e, "0") != 0;
     if (const char* e = std::getenv("LLM_ACCEL_TILE_FUSED"))
         c->tile_fused = std::strcmp(e, "0") != 0;
@@ -2263,6 +2282,205 @@ int run_stack(llm_ctx_t* c, const int16_t* rows_host, uint32_t rows, uint32_t po
     return 0;
 }
 
+// Rows of a prompt that go through a layer at once (its workspace is bounded
+// by them), and the blocks from which that is the faster way: one layer of
+// config B takes 51 us per 8-row block and ~145 us for 16 to 32 rows at once.
+constexpr uint32_t kPfMaxRows = 2048, kPfMinBlocks = 4;
+// Split-K scratch of its products: at most 256 workgroup parts of 128 x 128
+// 64-bit sums, and their arrival counters.
+constexpr size_t kPfPartBytes = (size_t)256 * 128 * 128 * 8;
+constexpr uint32_t kPfMaxTiles = 256;
+
+// Whether every matrix of layers [0, layer_count) has a layout that the
+// layer-major prompt path reads.
+bool prompt_path_ok(llm_ctx* c, uint32_t n_prompt, uint32_t block, uint32_t layer_count) {
+    if (!c->prompt_path || c->const_gain <= 0 || c->log_fn || cdiv(n_prompt, block) < kPfMinBlocks)
+        return false;
+    for (uint32_t l = 0; l < layer_count; l++) {
+        for (int m = 0; m < M_COUNT; m++) {
+            const Matrix& mt = c->mat(l, m);
+            if (mt.steps > llm::kP12MaxSteps || (!mt.p12_ok && !mt.mf)) return false;
+        }
+        const Matrix &g = c->mat(l, M_GATE), &u = c->mat(l, M_UP);
+        if (!(g.p12_ok && u.p12_ok) && !(g.mf && u.mf)) return false;
+    }
+    return true;
+}
+
+int prompt_buffers(llm_ctx* c, uint32_t rows) {
+    auto& p = c->pf;
+    const uint32_t R = round_up(rows, llm::kPfRowPad);
+    if (p.rows >= R) return 0;
+    if (p.base) {
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        if (int rc = dev_free(c, p.base)) return rc;
+        p = {};
+    }
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) / 256 * 256;
+        return o;
+    };
+    const uint32_t np = round_up(c->Nqkv, 128);
+    const size_t o_in = take((size_t)R * c->H * 2), o_ha = take((size_t)R * c->Hp * 2),
+                 o_hb = take((size_t)R * c->Hp * 2), o_qkv = take((size_t)R * np * 2),
+                 o_xn = take(llm::pf_xp_bytes(R, c->Hp)), o_xa = take(llm::pf_xp_bytes(R, c->Hp)),
+                 o_act = take(llm::pf_xp_bytes(R, c->Ip)),
+                 o_qp = take(llm::pf_qp_bytes(R, c->Hq, c->d)),
+                 o_kp = take(llm::pf_kp_bytes(c->Hkv, c->tiles, c->d)),
+                 o_vp = take(llm::pf_vp_bytes(c->Hkv, c->tiles, c->d)),
+                 o_kb = take((size_t)c->Hkv * c->tiles * 64 * 4), o_rs = take((size_t)R * 4),
+                 o_kf = take((size_t)2 * c->Hkv * c->tiles * 4),
+                 o_qf = take((size_t)c->Hq * (R / 32) * 4), o_ct = take(kPfMaxTiles * 4),
+                 o_pt = take(kPfPartBytes);
+    uint8_t* b = nullptr;
+    if (int rc = dev_alloc(c, (void**)&b, at)) return rc;
+    p.base = b;
+    p.in = (int16_t*)(b + o_in);
+    p.ha = (int16_t*)(b + o_ha);
+    p.hb = (int16_t*)(b + o_hb);
+    p.qkv = (int16_t*)(b + o_qkv);
+    p.xn = (int8_t*)(b + o_xn);
+    p.xa = (int8_t*)(b + o_xa);
+    p.act = (int8_t*)(b + o_act);
+    p.qp = (int8_t*)(b + o_qp);
+    p.kp = (int8_t*)(b + o_kp);
+    p.vp = (int8_t*)(b + o_vp);
+    p.kbias = (int32_t*)(b + o_kb);
+    p.rowsum = (int32_t*)(b + o_rs);
+    p.kvflag = (uint32_t*)(b + o_kf);
+    p.qflag = (uint32_t*)(b + o_qf);
+    p.count = (uint32_t*)(b + o_ct);
+    p.part = (int64_t*)(b + o_pt);
+    p.part_bytes = kPfPartBytes;
+    // attention outputs past the heads' width stay 0 (the attention writes
+    // whole heads only)
+    HIP_TRY(llm::launch_pf_init(p.in, R, 0, c->Hp, c->norms, c->const_gain, p.ha, p.xa, c->stream));
+    p.rows = R;
+    return 0;
+}
+
+// Prompt rows [0, n) (pinned host memory) through layers [0, layer_count),
+// layer by layer over up to kPfMaxRows rows at a time: K/V rows, hidden
+// pairs and final norm as the blocks of `block` rows leave them.
+int run_prompt_layers(llm_ctx* c, const int16_t* rows_host, uint32_t n, uint32_t block,
+                      uint32_t layer_count) {
+    hipStream_t st = c->stream;
+    const uint32_t chunk = std::min(n, kPfMaxRows / block * block);
+    if (int rc = prompt_buffers(c, chunk)) return rc;
+    auto& p = c->pf;
+    auto gemm = [&](const int8_t* x, uint32_t m, const Matrix& w, const Matrix* w2, int epi,
+                    const int16_t* res, int16_t* out, int8_t* xp, const int16_t* gamma) -> int {
+        llm::PfGemmArgs a{};
+        a.x = x;
+        a.m = m;
+        a.steps = w.steps;
+        a.n = w.n;
+        a.kq = w.kq;
+        a.ms0 = w.ms;
+        a.ms1 = w2 ? w2->ms : nullptr;
+        if (w.p12_ok && (!w2 || w2->p12_ok)) {
+            a.p0 = w.p12;
+            a.p1 = w2 ? w2->p12 : nullptr;
+            a.corr0 = w.corr_any ? w.corr : nullptr;
+            a.corr1 = w2 && w2->corr_any ? w2->corr : nullptr;
+        } else {
+            a.mf0 = w.mf;
+            a.mf1 = w2 ? w2->mf : nullptr;
+            HIP_TRY(llm::launch_pf_rowsum(x, m, w.steps, p.rowsum, st));
+            a.rowsum = p.rowsum;
+        }
+        a.res = res;
+        a.out = out;
+        a.xp_out = xp;
+        a.norm_gamma = gamma;
+        a.norm_gain = c->const_gain;
+        a.silu8 = c->silu8;
+        a.part = p.part;
+        a.part_bytes = p.part_bytes;
+        a.count = p.count;
+        a.max_tiles = kPfMaxTiles;
+        HIP_TRY(llm::launch_pf_gemm(a, epi, st));
+        return 0;
+    };
+    for (uint32_t c0 = 0; c0 < n; c0 += chunk) {
+        const uint32_t m = std::min(chunk, n - c0);
+        HIP_TRY(hipMemcpyAsync(p.in, rows_host + (size_t)c0 * c->H, (size_t)m * c->H * 2,
+                               hipMemcpyHostToDevice, st));
+        c->n_h2d_rows += cdiv(m, block);  // counted per block of rows
+        HIP_TRY(llm::launch_pf_init(p.in, m, c->H, c->Hp, c->norms, c->const_gain, p.ha, p.xn, st));
+        for (uint32_t l = 0; l < layer_count; l++) {
+            int rc = check_layer_loaded(c, l, true, true);
+            if (rc) return rc;
+            const int16_t* gf = c->norms + (size_t)(2 * l + 1) * c->H;
+            const int16_t* gn = c->norms + (size_t)(2 * l + 2) * c->H;
+            {
+                TimedScope ts(c, LLM_K_QKV);
+                if ((rc = gemm(p.xn, m, c->mat(l, M_QKV), nullptr, llm::EPI_STORE, nullptr, p.qkv,
+                               nullptr, nullptr)))
+                    return rc;
+            }
+            llm::PfAttnArgs at{};
+            at.qkv = p.qkv;
+            at.qkv_nt = round_up(c->Nqkv, 128) / 32;
+            at.m = m;
+            at.pos0 = c0;
+            at.rope = c->rope;
+            const size_t layer_off = (size_t)l * c->Hkv * c->tiles * llm::kTile * c->d;
+            at.kcache = c->kcache + layer_off;
+            at.vcache = c->vcache + layer_off;
+            at.tiles = c->tiles;
+            at.num_heads = c->Hq;
+            at.num_kv_heads = c->Hkv;
+            at.group = c->G;
+            at.head_dim = c->d;
+            at.qk_scale = c->qk_scale;
+            at.exp14 = c->exp14;
+            at.qp = p.qp;
+            at.kp = p.kp;
+            at.vp = p.vp;
+            at.kbias = p.kbias;
+            at.kvflag = p.kvflag;
+            at.qflag = p.qflag;
+            at.xp_out = p.xa;
+            at.out_steps = c->Hp / 128;
+            {
+                TimedScope ts(c, LLM_K_ROPE);
+                HIP_TRY(llm::launch_pf_kvq(at, st));
+            }
+            {
+                TimedScope ts(c, LLM_K_ATTENTION);
+                HIP_TRY(llm::launch_pf_attention(at, st));
+            }
+            {
+                TimedScope ts(c, LLM_K_OPROJ);
+                if ((rc = gemm(p.xa, m, c->mat(l, M_O), nullptr, llm::EPI_RESID, p.ha, p.hb, p.xn, gf)))
+                    return rc;
+            }
+            {
+                TimedScope ts(c, LLM_K_GATEUP);
+                if ((rc = gemm(p.xn, m, c->mat(l, M_GATE), &c->mat(l, M_UP), llm::EPI_SILU, nullptr,
+                               nullptr, p.act, nullptr)))
+                    return rc;
+            }
+            {
+                TimedScope ts(c, LLM_K_DOWN);
+                const bool next = l + 1 < layer_count;
+                if ((rc = gemm(p.act, m, c->mat(l, M_DOWN), nullptr, llm::EPI_RESID, p.hb, p.ha,
+                               next ? p.xn : nullptr, next ? gn : nullptr)))
+                    return rc;
+            }
+        }
+        invalidate_pair(c, 0);
+        invalidate_pair(c, 1);
+        HIP_TRY(llm::launch_pf_finish(p.hb, p.ha, m, c->H, c->Hp, block, c0 + m == n,
+                                      c->norms + (size_t)(2 * c->L) * c->H, c->const_gain,
+                                      c->pairs[0], c->pairs[1], st));
+    }
+    return 0;
+}
+
 // The LM-head argmax of rows [row0, row0 + rows) of `pair` enqueued, its
 // keys copied into pinned host memory; the caller synchronises.
 int ensure_keys_host(llm_ctx_t* c) {
@@ -2387,6 +2605,19 @@ int llm_generate(llm_ctx_t* c, const int16_t* embedding, uint32_t vocab,
     auto run_prompt = [&](bool count) -> int {
         uint32_t uncounted = 0;
         HIP_TRY(hipEventRecord(ev_p0, c->stream));
+        if (prompt_path_ok(c, n_prompt, block_size, layer_count)) {
+            if (int r = run_prompt_layers(c, c->stage, n_prompt, block_size, layer_count)) return r;
+            const uint32_t blocks = (uint32_t)cdiv(n_prompt, block_size);
+            if (count) {
+                S.coarse_task_count += blocks * 2 * layer_count + 1;
+                S.prompt_forward_passes = blocks;
+                S.output_materializations++;
+                S.released_prompt_blocks = blocks - 1;
+            }
+            last_row = (n_prompt - 1) % block_size;
+            HIP_TRY(hipEventRecord(ev_p1, c->stream));
+            return 0;
+        }
         for (uint32_t b0 = 0; b0 < n_prompt; b0 += block_size) {
             const uint32_t rows = std::min(block_size, n_prompt - b0);
             const bool final_block = b0 + rows == n_prompt;

@@ -1,0 +1,150 @@
+"""The layer-major prompt path of llm_generate (csrc/prefill.hip) against the
+block-by-block prompt, bit for bit: sampled tokens, every K/V row, both hidden
+pairs and the report's counts, over row counts at the edges of the 32-row pieces,
+64-position tiles and 64- / 128-row workgroup tiles, ragged block sizes, head_dims
+that fill the matrix cores' operands and that do not, 12-bit weights with and
+without corrections, 16-bit weights, and saturating queries, keys and values; and
+once against the oracle's block by block replay."""
+import sys
+
+import numpy as np
+import pytest
+
+import workloads
+from helpers import accel_shape, oracle_from_synthetic, oracle_shape
+
+pytestmark = pytest.mark.gpu
+
+# (vocab, hidden, inter, heads, KV heads): head_dim 64, 128, 48, 32 and 16
+D64 = workloads.ShapeSpec("d64", 512, 256, 688, 2, 4, 2, 1200, 0.25, 0.5)
+D128 = workloads.ShapeSpec("d128", 512, 1024, 1300, 2, 8, 2, 1200, 0.125, 0.3)
+D48 = workloads.ShapeSpec("d48", 512, 480, 1300, 2, 10, 2, 1200, 0.125, 0.3)
+D32 = workloads.ShapeSpec("d32", 512, 192, 260, 2, 6, 3, 1200, 0.25, 0.5)
+D16 = workloads.ShapeSpec("d16", 512, 128, 132, 2, 8, 8, 1200, 0.25, 0.5)
+
+
+def _say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+class Model:
+    """Arrays of a SyntheticModel with weights planted or replaced."""
+
+    def __init__(self, spec, kind):
+        self.synth = workloads.SyntheticModel(spec)
+        rng = np.random.default_rng(91)
+        self.emb = self.synth.embedding()
+        for layer in range(spec.layers):
+            for proj in range(7):
+                w = self.synth.weight(layer, proj)
+                n, k = w.shape
+                if kind == "corrections":
+                    for r in (0, 1, n // 2, n - 1):
+                        cols = rng.choice(k, size=4, replace=False)
+                        w[r, cols] = rng.choice([-32768, -2049, 2048, 30000], size=4)
+                elif kind == "wide":
+                    w[rng.random(w.shape) < 0.02] = 4095
+                    w[0, :6] = [32767, -32768, 32640, 32767, -2049, 2048]
+        if kind == "saturating":  # q, k, v past the Q4.12 operand's range
+            for proj in range(3):
+                self.synth.weight(0, proj)[:] = rng.integers(-2048, 2048, size=self.synth.weight(0, proj).shape)
+        if kind == "extreme":
+            # every query and key element of layer 0 the lowest value: at
+            # position 0 each bank's sum is exactly 2^31
+            self.emb = np.abs(self.emb) + 64
+            for proj in range(2):
+                self.synth.weight(0, proj)[:] = -2048
+
+    def weight(self, layer, proj):
+        return self.synth.weight(layer, proj)
+
+    def norms(self):
+        return self.synth.norms()
+
+
+def _request(monkeypatch, spec, model, prompt, block, gen, layer_major):
+    import llm_accel
+    monkeypatch.setenv("LLM_ACCEL_PROMPT", "1" if layer_major else "0")
+    with llm_accel.Accelerator(accel_shape(spec)) as a:
+        a.load_model(model)
+        a.load_lm_head(model.emb)
+        for pair in (0, 1):  # rows that no block writes stay what they were
+            a.upload(pair, np.full((8, spec.hidden), 7 + pair, np.int16))
+        toks, st = a.generate(model.emb, prompt, block, spec.layers, gen)
+        kv = [a.kv_read(layer, h, 0, len(prompt)) for layer in range(spec.layers)
+              for h in range(spec.kv_heads)]
+        pairs = [a.download(p, 8) for p in (0, 1)]
+        # the next tasks find the state a block left
+        a.task(18, 0, 1, len(prompt), 1, 0)
+        more = a.download(0, 8)
+    counts = {k: v for k, v in st.items() if not k.endswith("ms")}
+    return toks, kv, pairs, more, counts
+
+
+def _compare(monkeypatch, spec, kind, n, block, gen=1):
+    model = Model(spec, kind)
+    rng = np.random.default_rng(n)
+    prompt = [int(t) for t in rng.integers(0, spec.vocab, size=n)]
+    _say(f"case {spec.name} {kind} P{n} B{block}")
+    want = _request(monkeypatch, spec, model, prompt, block, gen, False)
+    got = _request(monkeypatch, spec, model, prompt, block, gen, True)
+    assert got[0] == want[0], "tokens"
+    for i, ((k0, v0), (k1, v1)) in enumerate(zip(want[1], got[1])):
+        assert np.array_equal(k0, k1), f"K rows {i}: {np.argwhere(k0 != k1)[:3]}"
+        assert np.array_equal(v0, v1), f"V rows {i}"
+    for p in (0, 1):
+        assert np.array_equal(got[2][p], want[2][p]), \
+            f"pair {p}: {np.argwhere(got[2][p] != want[2][p])[:3]}"
+    assert np.array_equal(got[3], want[3])
+    assert got[4] == want[4]
+
+
+@pytest.mark.parametrize("n,block", [(4, 1), (31, 8), (33, 5), (64, 8), (65, 8), (127, 3),
+                                     (129, 8), (200, 7)])
+def test_row_counts(monkeypatch, n, block):
+    _compare(monkeypatch, D64, "plain", n, block)
+
+
+@pytest.mark.parametrize("spec", [D128, D48, D32, D16], ids=lambda s: s.name)
+@pytest.mark.parametrize("n,block", [(26, 8), (193, 6)])
+def test_head_dims(monkeypatch, spec, n, block):
+    _compare(monkeypatch, spec, "plain", n, block, gen=3)
+
+
+@pytest.mark.parametrize("kind", ["corrections", "wide", "saturating", "extreme"])
+@pytest.mark.parametrize("spec", [D64, D128, D48], ids=lambda s: s.name)
+def test_weights_and_saturation(monkeypatch, spec, kind):
+    _compare(monkeypatch, spec, kind, 131, 8)
+
+
+def test_long_prompt(monkeypatch):
+    _compare(monkeypatch, D128, "plain", 1100, 8)
+
+
+def test_oracle_replay(monkeypatch):
+    """Hidden pairs and K/V rows of a prompt over three tiles against the
+    oracle's task by task replay."""
+    import llm_accel
+    spec, n, block = D64, 139, 8
+    model = Model(spec, "corrections")
+    prompt = [int(t) for t in np.random.default_rng(5).integers(0, spec.vocab, size=n)]
+    om = oracle_from_synthetic(model, oracle_shape(spec))
+    kv = om.new_kv()
+    for b0 in range(0, n, block):
+        h = model.emb[prompt[b0:b0 + block]].copy()
+        for layer in range(spec.layers):
+            _, h, _ = om.task(kv, 18, layer, h, b0)
+            _, h, _ = om.task(kv, 19, layer, h, b0)
+    _, fin, _ = om.task(kv, 20, 0, h, b0)
+    with llm_accel.Accelerator(accel_shape(spec)) as a:
+        a.load_model(model)
+        a.generate(model.emb, prompt, block, spec.layers, 0)
+        rows = n - b0
+        assert np.array_equal(a.download(1, rows), h)
+        assert np.array_equal(a.download(0, rows), fin)
+        for layer in range(spec.layers):
+            for hd in range(spec.kv_heads):
+                k, v = a.kv_read(layer, hd, 0, n)
+                assert np.array_equal(k, kv[0][layer, hd, :n]), f"K {layer} {hd}"
+                assert np.array_equal(v, kv[1][layer, hd, :n]), f"V {layer} {hd}"
