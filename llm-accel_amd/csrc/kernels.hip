@@ -1052,6 +1052,146 @@ __global__ __launch_bounds__(256) void lm_argmax_kernel(const int16_t* __restric
     }
 }
 
+// The same for blocks of 3-8 rows on the matrix cores: the VALU kernel's
+// products grow with the rows (8 rows of the 151,936 x 2,048 table: 400 us
+// against 116 for one, whose time is the table's bytes; here 120).  With w = 256 a + b
+// + 128 and x = 256 c + d + 128 (signed bytes),
+//   sum w x = 65536 sum ac + 256 (sum ad + sum bc) + sum bd
+//             + 128 sum (256 a + b) + 128 sum x,
+// all sums exact in int32 (hidden <= 3840 here): the MFMA's columns are the
+// eight rows' c and the eight rows' d, its other operand 16 table rows' a,
+// then b, and a product with ones gives sum a and sum b.  The activations
+// wait in LDS in operand order; a lane's table bytes are 8-column pieces
+// (columns 32 q + 8 g of a step), so that each load of a wavefront covers
+// 64 contiguous bytes of 16 rows.  A wavefront walks 16-row groups, or, for
+// tables of few groups (KS), the four wavefronts of a workgroup share one.
+constexpr uint32_t kLmGroup = 16;
+// Activations of at most 60 KiB (44 with the shared groups' sums) in LDS.
+constexpr uint32_t kLmMfmaSteps = 30, kLmMfmaStepsShared = 22;
+template <bool KS>
+__global__ __launch_bounds__(256) void lm_argmax_mfma_kernel(const int16_t* __restrict__ w,
+                                                             uint32_t S, uint32_t n,
+                                                             const int16_t* __restrict__ x,
+                                                             uint32_t ldx, uint32_t rows,
+                                                             unsigned long long* keys) {
+    extern __shared__ __attribute__((aligned(16))) int8_t lm_x[];  // [S][2][64][16]
+    __shared__ int32_t xsum[8];
+    __shared__ unsigned long long wbest[4][16];
+    __shared__ v4i red[KS ? 4 : 1][4][64];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t j = lane & 15, g = lane >> 4;
+    if (tid < 8) xsum[tid] = 0;
+    __syncthreads();
+    // thread: 8 columns of a row, as 8 bytes of c and of d
+    for (uint32_t e = tid; e < S * 128; e += 256) {
+        const uint32_t r = e & 7, k8 = e >> 3;  // row, 8-column piece
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (r < rows) v = *(const uint4*)(x + (size_t)r * ldx + 8 * k8);
+        const uint32_t s = k8 >> 4, q = (k8 >> 2) & 3, gg = k8 & 3;
+        int8_t* o = lm_x + ((s * 2 + (q >> 1)) * 64 + r + 16 * gg) * 16 + 8 * (q & 1);
+        typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+        *(v2u*)o = v2u{__builtin_amdgcn_perm(v.y, v.x, 0x07050301u),
+                       __builtin_amdgcn_perm(v.w, v.z, 0x07050301u)};
+        *(v2u*)(o + 8 * 16) = v2u{__builtin_amdgcn_perm(v.y, v.x, 0x06040200u) ^ 0x80808080u,
+                                  __builtin_amdgcn_perm(v.w, v.z, 0x06040200u) ^ 0x80808080u};
+        int32_t t = dot2(v.x, 0x00010001u, 0);
+        t = dot2(v.y, 0x00010001u, t);
+        t = dot2(v.z, 0x00010001u, t);
+        t = dot2(v.w, 0x00010001u, t);
+        if (r < rows) atomicAdd(&xsum[r], t);
+    }
+    __syncthreads();
+    const uint32_t ngroups = (n + kLmGroup - 1) / kLmGroup, nblk = (n + 3) / 4;
+    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    const uint32_t s0 = KS ? wave * S / 4 : 0, s1 = KS ? (wave + 1) * S / 4 : S;
+    const uint32_t first = KS ? blockIdx.x : blockIdx.x * 4 + wave;
+    const uint32_t stride = KS ? gridDim.x : gridDim.x * 4;
+    unsigned long long best = 0;
+    for (uint32_t gr = first; gr < ngroups; gr += stride) {
+        // row 16 gr + j: block 4 gr + j / 4 (clamped: rows past n are not used)
+        const uint32_t blk = min(4 * gr + (j >> 2), nblk - 1);
+        const int16_t* wp = w + ((size_t)blk * S * 4 + (j & 3)) * 128 + 8 * g;
+        v4u buf[2][4];
+        auto load = [&](int set, uint32_t s) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) buf[set][q] = *(const v4u*)(wp + (size_t)s * 512 + 32 * q);
+        };
+        v4i ha = {0, 0, 0, 0}, la = ha, sa = ha, sb = ha;  // a x, b x, a, b
+        auto step = [&](int set, uint32_t s) {
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const v4u u = buf[set][2 * c], v = buf[set][2 * c + 1];
+                const v4i a = {(int32_t)__builtin_amdgcn_perm(u.y, u.x, 0x07050301u),
+                               (int32_t)__builtin_amdgcn_perm(u.w, u.z, 0x07050301u),
+                               (int32_t)__builtin_amdgcn_perm(v.y, v.x, 0x07050301u),
+                               (int32_t)__builtin_amdgcn_perm(v.w, v.z, 0x07050301u)};
+                v4i b = {(int32_t)__builtin_amdgcn_perm(u.y, u.x, 0x06040200u),
+                         (int32_t)__builtin_amdgcn_perm(u.w, u.z, 0x06040200u),
+                         (int32_t)__builtin_amdgcn_perm(v.y, v.x, 0x06040200u),
+                         (int32_t)__builtin_amdgcn_perm(v.w, v.z, 0x06040200u)};
+                b ^= v4i{(int32_t)0x80808080u, (int32_t)0x80808080u, (int32_t)0x80808080u,
+                         (int32_t)0x80808080u};
+                const v4i xv = *(const v4i*)(lm_x + ((s * 2 + c) * 64 + lane) * 16);
+                ha = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, xv, ha, 0, 0, 0);
+                la = __builtin_amdgcn_mfma_i32_16x16x64_i8(b, xv, la, 0, 0, 0);
+                sa = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ones, sa, 0, 0, 0);
+                sb = __builtin_amdgcn_mfma_i32_16x16x64_i8(b, ones, sb, 0, 0, 0);
+            }
+        };
+        if (s0 < s1) {
+            load(0, s0);
+            for (uint32_t s = s0; s < s1; s += 2) {
+                load(1, s + 1 < s1 ? s + 1 : s);
+                step(0, s);
+                load(0, s + 2 < s1 ? s + 2 : s);
+                if (s + 1 < s1) step(1, s + 1);
+            }
+        }
+        if constexpr (KS) {
+            red[wave][0][lane] = ha;
+            red[wave][1][lane] = la;
+            red[wave][2][lane] = sa;
+            red[wave][3][lane] = sb;
+            __syncthreads();
+            if (wave == 0) {
+#pragma unroll
+                for (int q = 1; q < 4; q++) {
+                    ha += red[q][0][lane];
+                    la += red[q][1][lane];
+                    sa += red[q][2][lane];
+                    sb += red[q][3][lane];
+                }
+            }
+            __syncthreads();
+        }
+        // lane (j, g) holds table rows 16 gr + 4 g + t: column j < 8 the sums
+        // with row j's c, column j + 8 those with its d
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int32_t ad = __builtin_amdgcn_update_dpp(0, ha[t], 0x128, 0xf, 0xf, false);
+            const int32_t bd = __builtin_amdgcn_update_dpp(0, la[t], 0x128, 0xf, 0xf, false);
+            const int64_t score = 65536 * (int64_t)ha[t] + 256 * ((int64_t)ad + la[t]) + bd +
+                                  128 * (256 * (int64_t)sa[t] + sb[t] + xsum[j & 7]);
+            const uint32_t v = kLmGroup * gr + 4 * g + t;
+            const unsigned long long k = argmax_key(score, v);
+            if (v < n && k > best) best = k;
+        }
+    }
+    // the best of a row's lanes (g), then of the wavefronts
+#pragma unroll
+    for (int o = 16; o < 64; o *= 2) {
+        const unsigned long long k = __shfl_xor(best, o);
+        best = k > best ? k : best;
+    }
+    if (lane < 8) wbest[wave][lane] = best;
+    __syncthreads();
+    if (tid < 8 && tid < rows) {
+        unsigned long long k = 0;
+        for (int q = 0; q < (KS ? 1 : 4); q++) k = wbest[q][tid] > k ? wbest[q][tid] : k;
+        atomicMax(&keys[tid], k);
+    }
+}
+
 template <int RT>
 static hipError_t launch_lm_rt(const int16_t* w, uint32_t steps, uint32_t n,
                                const int16_t* x, uint32_t ldx, uint32_t rows, int L,
@@ -1083,6 +1223,22 @@ static hipError_t launch_lm_rt(const int16_t* w, uint32_t steps, uint32_t n,
 hipError_t launch_lm_argmax(const int16_t* w, uint32_t steps, uint32_t n,
                             const int16_t* x, uint32_t ldx, uint32_t rows, int L,
                             unsigned long long* keys, hipStream_t st) {
+    // From three rows on the matrix cores (call times at hidden 2048, 151,936
+    // rows: 3 rows 236 -> 135 us, 5 410 -> 135, 8 415 -> 134; one and two
+    // rows 122 and 128 us against 134).  Tables of fewer groups than 2,048
+    // wavefronts can walk share each among a workgroup's wavefronts; larger
+    // ones take one workgroup per compute unit (512 and 1,024 workgroups:
+    // 153 and 139 us, their last round nearly empty).
+    const uint32_t groups = (n + kLmGroup - 1) / kLmGroup;
+    const bool shared = groups < 2048;
+    if (rows >= 3 && steps <= (shared ? kLmMfmaStepsShared : kLmMfmaSteps)) {
+        const uint32_t lds = steps * 2048;
+        if (shared)
+            lm_argmax_mfma_kernel<true><<<groups, 256, lds, st>>>(w, steps, n, x, ldx, rows, keys);
+        else
+            lm_argmax_mfma_kernel<false><<<256, 256, lds, st>>>(w, steps, n, x, ldx, rows, keys);
+        return hipGetLastError();
+    }
     if (rows <= 1) return launch_lm_rt<1>(w, steps, n, x, ldx, rows, L, keys, st);
     if (rows <= 2) return launch_lm_rt<2>(w, steps, n, x, ldx, rows, L, keys, st);
     if (rows <= 4) return launch_lm_rt<4>(w, steps, n, x, ldx, rows, L, keys, st);
