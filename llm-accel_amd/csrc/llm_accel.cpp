@@ -225,6 +225,7 @@ struct llm_ctx {
     int16_t* ports[3] = {nullptr, nullptr, nullptr};
     size_t port_n = 0;                  // elements per port
     int16_t* op_stage = nullptr;        // [8][max(Hp, Ip)]
+    int32_t* op_tsum = nullptr;         // tile sums of the operator-level flash attention
     // partial sums / arrival counters of the split matrix-core projection
     int32_t* mf_part = nullptr;
     uint32_t* mf_count = nullptr;
@@ -1658,6 +1659,8 @@ int ensure_ports(llm_ctx* c) {
         if (int rc = dev_alloc(c, (void**)&c->op_stage,
                                (size_t)8 * std::max(c->Hp, c->Ip) * 2))
             return rc;
+    if (!c->op_tsum)
+        if (int rc = dev_alloc(c, (void**)&c->op_tsum, c->rht_words * 4)) return rc;
     c->port_n = n;
     c->ports_ready = true;
     return 0;
@@ -1867,6 +1870,10 @@ int llm_op(llm_ctx_t* c, uint32_t op, uint32_t layer, uint32_t token_count,
         fa.exp14 = c->exp14;
         fa.legacy = block ? 0 : 1;
         fa.out = out;
+        fa.s_scores = c->s_scores;
+        fa.s_tmax = c->s_tmax;
+        fa.s_tsum = c->op_tsum;
+        fa.s_tval = c->s_tval;
         HIP_TRY(llm::launch_op_flash(fa, s));
     }
     fill_op_counters(c, op, T, position, tile_len, st);

@@ -53,6 +53,13 @@ struct OpFlashArgs {
     const int16_t* exp14;
     int legacy;
     int16_t* out;
+    // scratch of the tile-parallel launches, per (token, KV head, tile,
+    // query head), tile stride `tiles`: scores, their maximum, the
+    // probabilities' sum, the PV values
+    int16_t* s_scores;  // [8][kv_heads][tiles][group][64]
+    int16_t* s_tmax;    // [8][kv_heads][tiles][group]
+    int32_t* s_tsum;    // [8][kv_heads][tiles][group]
+    int16_t* s_tval;    // [8][kv_heads][tiles][group][head_dim]
 };
 hipError_t launch_op_flash(const OpFlashArgs& a, hipStream_t st);
 // Writes k[h] / v[h] (head_dim each) as position pos of every KV head's
