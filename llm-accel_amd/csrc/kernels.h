@@ -106,6 +106,17 @@ __device__ __forceinline__ unsigned long long argmax_key(int64_t score, uint32_t
     return ((unsigned long long)(score + ((int64_t)1 << 45)) << 18) |
            (unsigned long long)(kArgmaxVocabMax - v);
 }
+// Publishes the argmax keys of 8 rows to host_keys (pinned host memory) and
+// clears them for the next argmax, then stores seq to *flag (pinned).
+hipError_t launch_keys_out(unsigned long long* keys, unsigned long long* host_keys, uint32_t* flag,
+                           uint32_t seq, hipStream_t st);
+// `rows` rows of `cols` int16 between device memory and pinned host memory,
+// or within device memory (addresses 16-byte aligned; row strides in
+// elements; cols and strides multiples of 8, or one row of any length).  With a flag (pinned), seq is stored there once every value
+// is visible to the host; count is a device word that is 0 between launches.
+hipError_t launch_io_rows(const int16_t* src, uint32_t ld_src, int16_t* dst, uint32_t ld_dst,
+                          uint32_t cols, uint32_t rows, uint32_t* count, uint32_t* flag,
+                          uint32_t seq, hipStream_t st);
 hipError_t launch_lm_argmax(const int16_t* w, uint32_t steps, uint32_t n,
                             const int16_t* x, uint32_t ldx, uint32_t rows, int L,
                             unsigned long long* keys, hipStream_t st);

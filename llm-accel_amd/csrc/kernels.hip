@@ -1246,6 +1246,73 @@ hipError_t launch_lm_argmax(const int16_t* w, uint32_t steps, uint32_t n,
 }
 
 // ---------------------------------------------------------------------
+// Small transfers with the host, by kernels over pinned memory: a pageable
+// copy of 8 rows of 2,048 took ~70 us in the runtime either way, a pinned
+// one ~10 us and a wait ~10 us; a kernel reads or writes the 32 KiB over
+// the bus in 3-4 us, and the host polls a word that the kernel stores last
+// instead of waiting for the stream.
+// ---------------------------------------------------------------------
+// A thread's values become visible to the host before the flag: each
+// workgroup fences its stores at system scope before it arrives (stores
+// that each go through the caches instead, 8 bytes at a time, took 650 us for
+// 172 KiB).
+__device__ __forceinline__ void publish(uint32_t* count, uint32_t* flag, uint32_t seq) {
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    if (gridDim.x > 1) {
+        const uint32_t prev = __hip_atomic_fetch_add(count, 1u, __ATOMIC_ACQ_REL,
+                                                     __HIP_MEMORY_SCOPE_AGENT);
+        if (prev != gridDim.x - 1) return;
+        __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Thread: 16 bytes (a thread of four pieces took 7 us for 32 KiB instead of
+// 3.5: the bus wants many wavefronts).
+__global__ __launch_bounds__(256) void io_rows_kernel(const int16_t* __restrict__ src,
+                                                      uint32_t ld_src, int16_t* __restrict__ dst,
+                                                      uint32_t ld_dst, uint32_t cols, uint32_t n,
+                                                      uint32_t* count, uint32_t* flag,
+                                                      uint32_t seq) {
+    const uint32_t c8 = (cols + 7) / 8;  // pieces of a row; n: of all rows
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) {
+        const uint32_t r = i / c8, c = 8 * (i % c8);
+        if (c + 8 <= cols)
+            *(uint4*)(dst + (size_t)r * ld_dst + c) = *(const uint4*)(src + (size_t)r * ld_src + c);
+        else  // the end of a single row
+            for (uint32_t e = c; e < cols; e++) dst[e] = src[e];
+    }
+    if (flag) publish(count, flag, seq);
+}
+
+hipError_t launch_io_rows(const int16_t* src, uint32_t ld_src, int16_t* dst, uint32_t ld_dst,
+                          uint32_t cols, uint32_t rows, uint32_t* count, uint32_t* flag,
+                          uint32_t seq, hipStream_t st) {
+    if (rows > 1 && (cols % 8 || ld_src % 8 || ld_dst % 8)) return hipErrorInvalidValue;
+    const uint32_t n = (cols + 7) / 8 * rows, grid = n ? (n + 255) / 256 : 1;
+    io_rows_kernel<<<grid, 256, 0, st>>>(src, ld_src, dst, ld_dst, cols, n, count, flag, seq);
+    return hipGetLastError();
+}
+
+__global__ __launch_bounds__(64) void keys_out_kernel(unsigned long long* keys,
+                                                      unsigned long long* host_keys,
+                                                      uint32_t* flag, uint32_t seq) {
+    if (threadIdx.x < 8) {
+        host_keys[threadIdx.x] = keys[threadIdx.x];
+        keys[threadIdx.x] = 0;
+    }
+    publish(nullptr, flag, seq);
+}
+hipError_t launch_keys_out(unsigned long long* keys, unsigned long long* host_keys, uint32_t* flag,
+                           uint32_t seq, hipStream_t st) {
+    keys_out_kernel<<<1, 64, 0, st>>>(keys, host_keys, flag, seq);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------
 // Plain copy (calibration reference for HBM counters).
 // ---------------------------------------------------------------------
 __global__ __launch_bounds__(256) void copy_kernel(const uint4* __restrict__ src,

@@ -221,7 +221,7 @@ struct llm_ctx {
     int16_t* xn_final = nullptr;        // [8][Hp]
     // Operator-level commands (llm_op): the context's own in / aux / out
     // port buffers and the 8-row projection staging, allocated on first use.
-    bool ports_ready = false;
+    bool ports_ready = false, port_out = false;
     int16_t* ports[3] = {nullptr, nullptr, nullptr};
     size_t port_n = 0;                  // elements per port
     int16_t* op_stage = nullptr;        // [8][max(Hp, Ip)]
@@ -272,6 +272,21 @@ struct llm_ctx {
         size_t part_bytes = 0;
     } pf;
     bool prompt_path = true;
+    // Transfers of rows and keys with the host: pinned staging (in: host to
+    // device, out: device to host), the pinned word a transfer's kernel sets
+    // to its number once its values are visible, and a device word for its
+    // workgroups' arrivals.  `busy`: what has been enqueued since a transfer
+    // or synchronisation was last seen to complete (not relied on once the
+    // stream was handed out).
+    int16_t *io_in = nullptr, *io_out = nullptr;
+    size_t io_elems = 0;
+    uint32_t* io_flag = nullptr;
+    uint32_t* io_count = nullptr;
+    uint32_t io_seq = 0;
+    enum Busy { QUIET, COPIES_IN, WORK };
+    Busy busy = WORK;
+    bool stream_out = false;
+    size_t io_used = 0;   // of io_in, by copies not known to be complete
     uint64_t n_h2d_rows = 0;   // hidden-row uploads (calls)
     uint64_t n_d2h_rows = 0;   // hidden-row downloads (calls)
     uint64_t n_kv_moves = 0;   // KV reads / writes (calls)
@@ -347,10 +362,110 @@ bool clear_waits(llm_ctx* c) {
 }
 
 // The same, reported as an error of the call that synchronised.
-int check_waits(llm_ctx* c) {
-    if (!clear_waits(c)) return 0;
+int late_error();
+int check_waits(llm_ctx* c) { return clear_waits(c) ? late_error() : 0; }
+
+int io_wait(llm_ctx* c, uint32_t seq);
+int ensure_keys_host(llm_ctx* c);
+
+// Everything enqueued so far has completed; `late` receives whether a
+// bounded wait gave up since the last time that was seen.
+int quiesce(llm_ctx* c, bool* late) {
+    *late = false;
+    if (c->busy == llm_ctx::QUIET && !c->stream_out) return 0;
+    const uint32_t seq = ++c->io_seq;  // an empty transfer
+    HIP_TRY(llm::launch_io_rows(nullptr, 0, nullptr, 0, 0, 0, c->io_count, c->io_flag, seq,
+                                c->stream));
+    if (int rc = io_wait(c, seq)) return rc;
+    *late = clear_waits(c);
+    return 0;
+}
+int late_error() {
     return fail(LLM_E_HIP, "a wait between workgroups of a fused launch timed out; "
                            "results since the last synchronisation are invalid");
+}
+
+// One port holds the largest tensor an operator exchanges: 8 feature rows
+// of the hidden or intermediate width, every KV head's K / V panel of 64
+// positions, or 64 scores per query head.
+size_t port_elems(const llm_ctx* c) {
+    return std::max({(size_t)8 * c->Hp, (size_t)8 * c->Ip, (size_t)64 * c->Hq, (size_t)64 * c->Ckv});
+}
+
+// Staging of at least `elems` int16 each way (made for the ports' size when
+// the context is created).
+int io_buffers(llm_ctx* c, size_t elems) {
+    if (c->io_elems >= elems) return 0;
+    HIP_TRY(hipStreamSynchronize(c->stream));  // a transfer may still read it
+    if (c->io_in) (void)hipHostFree(c->io_in);
+    c->io_in = c->io_out = nullptr;
+    c->io_elems = 0;
+    elems = (2 * elems + 2047) / 2048 * 2048;  // the two operands of a command
+    if (hipHostMalloc((void**)&c->io_in, 2 * elems * 2, hipHostMallocDefault) != hipSuccess)
+        return fail(LLM_E_NOMEM, "hipHostMalloc failed");
+    c->io_out = c->io_in + elems;
+    c->io_elems = elems;
+    return 0;
+}
+
+// Waits until transfer `seq` (the last work enqueued) is complete: polls
+// its word for a while, then leaves the wait to the runtime.
+int io_wait(llm_ctx* c, uint32_t seq) {
+    for (uint32_t i = 0; i < 200000; i++) {
+        if (__atomic_load_n(c->io_flag, __ATOMIC_ACQUIRE) == seq) {
+            c->busy = llm_ctx::QUIET;
+            return 0;
+        }
+        __builtin_ia32_pause();
+    }
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (__atomic_load_n(c->io_flag, __ATOMIC_ACQUIRE) != seq)
+        return fail(LLM_E_HIP, "a transfer to the host did not complete");
+    c->busy = llm_ctx::QUIET;
+    return 0;
+}
+
+// Rows of `cols` values from host memory into device rows: staged, the copy
+// enqueued and, unless `wait`, not waited for.
+int rows_in(llm_ctx* c, const int16_t* host, int16_t* dev, uint32_t ld_dev, uint32_t cols,
+            uint32_t rows, bool wait) {
+    bool late = false;
+    const size_t n = (size_t)rows * cols;
+    if (c->busy == llm_ctx::COPIES_IN && !c->stream_out && c->io_used + n <= c->io_elems) {
+        // only such copies are under way, and the staging has room
+    } else {
+        if (int rc = quiesce(c, &late)) return rc;
+        c->io_used = 0;
+    }
+    if (n) {
+        if (int rc = io_buffers(c, n)) return rc;
+        int16_t* from = c->io_in + c->io_used;
+        std::memcpy(from, host, n * 2);
+        c->io_used += (n + 7) / 8 * 8;
+        HIP_TRY(llm::launch_io_rows(from, cols, dev, ld_dev, cols, rows, nullptr, nullptr, 0,
+                                    c->stream));
+        c->busy = llm_ctx::COPIES_IN;
+        if (wait) HIP_TRY(hipStreamSynchronize(c->stream));
+    }
+    return late ? late_error() : 0;
+}
+
+// The same from the device, complete on return, with everything enqueued
+// before it.
+int rows_out(llm_ctx* c, const int16_t* dev, uint32_t ld_dev, int16_t* host, uint32_t cols,
+             uint32_t rows) {
+    if (rows && cols) {
+        if (int rc = io_buffers(c, (size_t)rows * cols)) return rc;
+        const uint32_t seq = ++c->io_seq;
+        HIP_TRY(llm::launch_io_rows(dev, ld_dev, c->io_out, cols, cols, rows, c->io_count,
+                                    c->io_flag, seq, c->stream));
+        if (int rc = io_wait(c, seq)) return rc;
+        std::memcpy(host, c->io_out, (size_t)rows * cols * 2);
+        return check_waits(c);
+    }
+    bool late;
+    if (int rc = quiesce(c, &late)) return rc;
+    return late ? late_error() : 0;
 }
 
 // While in scope, the context enqueues only launches whose workgroups never
@@ -1217,6 +1332,11 @@ int llm_ctx_create(const llm_shape_t* shape, int device, uint32_t num_pairs,
     if (hipHostMalloc((void**)&c->host_abort, 64, hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(LLM_E_NOMEM, "hipHostMalloc failed"));
     *c->host_abort = 0;
+    c->io_flag = c->host_abort + 8;  // a word of the same 64 bytes
+    *c->io_flag = 0;
+    if ((rc = dev_alloc(c, (void**)&c->io_count, 256)) || (rc = io_buffers(c, port_elems(c))) ||
+        (rc = ensure_keys_host(c)))
+        return cleanup(rc);
     if (const char* e = std::getenv("LLM_ACCEL_FUSED")) c->fused = std::strcmp(e, "0") != 0;
     if (const char* e = std::getenv("LLM_ACCEL_PROMPT"))
         c->prompt_path = std::strcmp(e, "0") != 0;
@@ -1309,6 +1429,7 @@ void llm_ctx_destroy(llm_ctx_t* c) {
     for (void* p : c->allocations) (void)hipFree(p);
     if (c->host_abort) (void)hipHostFree(c->host_abort);
     if (c->stage) (void)hipHostFree(c->stage);
+    if (c->io_in) (void)hipHostFree(c->io_in);
     if (c->keys_host) (void)hipHostFree(c->keys_host);
     for (auto e : c->gen_events) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1510,12 +1631,9 @@ int llm_hidden_upload(llm_ctx_t* c, uint32_t pair, const int16_t* rows,
         return fail(LLM_E_ARG, "bad hidden upload arguments");
     HIP_TRY(hipSetDevice(c->device));
     invalidate_pair(c, (int)pair);
-    HIP_TRY(hipMemcpy2DAsync(c->pairs[pair], (size_t)c->Hp * 2, rows,
-                             (size_t)c->H * 2, (size_t)c->H * 2, n,
-                             hipMemcpyHostToDevice, c->stream));
     c->n_h2d_rows++;
-    SYNC_TRY(c);
-    return 0;
+    // a pair whose address was handed out may be read on another stream
+    return rows_in(c, rows, c->pairs[pair], c->Hp, c->H, n, c->exported[pair]);
 }
 
 int llm_hidden_download(llm_ctx_t* c, uint32_t pair, int16_t* rows,
@@ -1523,12 +1641,8 @@ int llm_hidden_download(llm_ctx_t* c, uint32_t pair, int16_t* rows,
     if (!c || !rows || pair >= c->pairs.size() || n > 8)
         return fail(LLM_E_ARG, "bad hidden download arguments");
     HIP_TRY(hipSetDevice(c->device));
-    HIP_TRY(hipMemcpy2DAsync(rows, (size_t)c->H * 2, c->pairs[pair],
-                             (size_t)c->Hp * 2, (size_t)c->H * 2, n,
-                             hipMemcpyDeviceToHost, c->stream));
     c->n_d2h_rows++;
-    SYNC_TRY(c);
-    return 0;
+    return rows_out(c, c->pairs[pair], c->Hp, rows, c->H, n);
 }
 
 int llm_hidden_upload_ports(llm_ctx_t* c, uint32_t pair, const int16_t* port0,
@@ -1584,6 +1698,7 @@ int llm_task(llm_ctx_t* c, uint32_t op, uint32_t layer, uint32_t token_count,
     if (op > LLM_OP_FINAL_NORM) return reject(LLM_STATUS_BAD_OPERATOR);
     if (op == LLM_OP_NOP) return LLM_STATUS_OK;
     if (layer >= c->L) return reject(LLM_STATUS_BAD_LAYER);
+    c->busy = llm_ctx::WORK;
     const int ip = (int)in_pair, opr = (int)out_pair;
     if (hipSetDevice(c->device) != hipSuccess)
         return fail(LLM_E_HIP, "hipSetDevice failed");
@@ -1645,13 +1760,9 @@ namespace {
 // :1556-1675).
 // ---------------------------------------------------------------------
 
-// One port holds the largest tensor an operator exchanges: 8 feature rows
-// of the hidden or intermediate width, every KV head's K / V panel of 64
-// positions, or 64 scores per query head.
 int ensure_ports(llm_ctx* c) {
     if (c->ports_ready) return 0;
-    const size_t n = std::max({(size_t)8 * c->Hp, (size_t)8 * c->Ip, (size_t)64 * c->Hq,
-                               (size_t)64 * c->Ckv});
+    const size_t n = port_elems(c);
     for (int i = 0; i < 3; i++)
         if (!c->ports[i])
             if (int rc = dev_alloc(c, (void**)&c->ports[i], n * 2)) return rc;
@@ -1715,8 +1826,12 @@ int enqueue_op_projection(llm_ctx* c, uint32_t layer, uint32_t proj, uint32_t T,
     const uint32_t row0 = proj == 1 ? c->H : proj == 2 ? c->H + c->Ckv : 0;
     const uint32_t n = proj == 0 ? c->H : (proj <= 2 ? c->Ckv : m.n);
     if (T == 0) return 0;
-    HIP_TRY(hipMemcpy2DAsync(c->op_stage, (size_t)m.k_pad * 2, in, (size_t)m.k * 2,
-                             (size_t)m.k * 2, T, hipMemcpyDeviceToDevice, c->stream));
+    if (m.k % 8 == 0 && (uintptr_t)in % 16 == 0)  // what the copy kernel's loads need
+        HIP_TRY(llm::launch_io_rows(in, m.k, c->op_stage, m.k_pad, m.k, T, nullptr, nullptr, 0,
+                                    c->stream));
+    else
+        HIP_TRY(hipMemcpy2DAsync(c->op_stage, (size_t)m.k_pad * 2, in, (size_t)m.k * 2,
+                                 (size_t)m.k * 2, T, hipMemcpyDeviceToDevice, c->stream));
     llm::ProjArgs a{};
     a.w0 = m.d ? m.d + (size_t)row0 * m.k_pad : nullptr;
     a.steps = m.steps;
@@ -1748,7 +1863,10 @@ int llm_port(llm_ctx_t* c, uint32_t port, void** dev, size_t* elems) {
     if (!c || port > LLM_PORT_OUT) return fail(LLM_E_ARG, "bad port arguments");
     HIP_TRY(hipSetDevice(c->device));
     if (int rc = ensure_ports(c)) return rc;
-    if (dev) *dev = c->ports[port];
+    if (dev) {
+        *dev = c->ports[port];
+        c->port_out = true;  // port writes stay complete on return
+    }
     if (elems) *elems = c->port_n;
     return 0;
 }
@@ -1758,11 +1876,7 @@ int llm_port_write(llm_ctx_t* c, uint32_t port, const int16_t* host, size_t elem
     HIP_TRY(hipSetDevice(c->device));
     if (int rc = ensure_ports(c)) return rc;
     if (elems > c->port_n) return fail(LLM_E_ARG, "port write exceeds the port");
-    if (elems)
-        HIP_TRY(hipMemcpyAsync(c->ports[port], host, elems * 2, hipMemcpyHostToDevice,
-                               c->stream));
-    SYNC_TRY(c);
-    return 0;
+    return rows_in(c, host, c->ports[port], (uint32_t)elems, (uint32_t)elems, 1, c->port_out);
 }
 
 int llm_port_read(llm_ctx_t* c, uint32_t port, int16_t* host, size_t elems) {
@@ -1770,11 +1884,7 @@ int llm_port_read(llm_ctx_t* c, uint32_t port, int16_t* host, size_t elems) {
     HIP_TRY(hipSetDevice(c->device));
     if (int rc = ensure_ports(c)) return rc;
     if (elems > c->port_n) return fail(LLM_E_ARG, "port read exceeds the port");
-    if (elems)
-        HIP_TRY(hipMemcpyAsync(host, c->ports[port], elems * 2, hipMemcpyDeviceToHost,
-                               c->stream));
-    SYNC_TRY(c);
-    return 0;
+    return rows_out(c, c->ports[port], (uint32_t)elems, host, (uint32_t)elems, 1);
 }
 
 int llm_op(llm_ctx_t* c, uint32_t op, uint32_t layer, uint32_t token_count,
@@ -1829,6 +1939,7 @@ int llm_op(llm_ctx_t* c, uint32_t op, uint32_t layer, uint32_t token_count,
     if (!in) in = c->ports[LLM_PORT_IN];
     if (!aux) aux = c->ports[LLM_PORT_AUX];
     if (!out) out = c->ports[LLM_PORT_OUT];
+    c->busy = llm_ctx::WORK;
     hipStream_t s = c->stream;
     const size_t layer_off = (size_t)layer * c->Hkv * c->tiles * llm::kTile * D;
     if (op <= LLM_OP_FFN_DOWN) {
@@ -1953,6 +2064,7 @@ int llm_kv_write(llm_ctx_t* c, uint32_t layer, uint32_t h, uint32_t pos0,
 
 int llm_kv_clear(llm_ctx_t* c) {
     if (!c) return fail(LLM_E_ARG, "null context");
+    c->busy = llm_ctx::WORK;
     HIP_TRY(hipSetDevice(c->device));
     const size_t bytes = (size_t)c->L * c->Hkv * c->tiles * 64 * c->d * 2;
     HIP_TRY(hipMemsetAsync(c->kcache, 0, bytes, c->stream));
@@ -1971,20 +2083,22 @@ void* llm_pair_device_ptr(llm_ctx_t* c, uint32_t pair) {
 
 void* llm_stream(llm_ctx_t* c) {
     if (!c) return nullptr;
-    // work collected for a persistent launch goes onto the stream first
     if (hipSetDevice(c->device) != hipSuccess) return nullptr;
+    c->stream_out = true;  // the caller may enqueue on it
     return (void*)c->stream;
 }
 
 int llm_sync(llm_ctx_t* c) {
     if (!c) return fail(LLM_E_ARG, "null context");
     HIP_TRY(hipSetDevice(c->device));
-    SYNC_TRY(c);
-    return 0;
+    bool late;
+    if (int rc = quiesce(c, &late)) return rc;
+    return late ? late_error() : 0;
 }
 
 int llm_event_record(llm_ctx_t* c, uint32_t slot) {
     if (!c || slot >= 1024) return fail(LLM_E_ARG, "bad event slot");
+    c->busy = llm_ctx::WORK;
     HIP_TRY(hipSetDevice(c->device));
     if (c->events.empty()) {
         c->events.resize(1024);
@@ -2004,6 +2118,7 @@ int llm_event_elapsed_ms(llm_ctx_t* c, uint32_t a, uint32_t b, float* ms) {
 
 int llm_kernel_timing(llm_ctx_t* c, int enable) {
     if (!c) return fail(LLM_E_ARG, "null context");
+    c->busy = llm_ctx::WORK;
     HIP_TRY(hipSetDevice(c->device));
     harvest_timing(c);
     for (int k = 0; k < LLM_K_COUNT; k++) c->kernel_ms[k] = 0, c->kernel_n[k] = 0;
@@ -2029,6 +2144,7 @@ int llm_bench_projection(llm_ctx_t* c, uint32_t kernel, uint32_t rows,
     if (kernel != LLM_K_QKV && kernel != LLM_K_OPROJ &&
         kernel != LLM_K_GATEUP && kernel != LLM_K_DOWN)
         return fail(LLM_E_ARG, "not a projection kernel");
+    c->busy = llm_ctx::WORK;
     HIP_TRY(hipSetDevice(c->device));
     auto launch = [&](uint32_t layer) -> hipError_t {
         llm::ProjArgs a{};
@@ -2105,6 +2221,7 @@ int llm_weight_bytes(llm_ctx_t* c, uint64_t* bytes, uint32_t* wide_matrices) {
 int llm_bench_copy(llm_ctx_t* c, uint64_t bytes, uint32_t iters, float* ms) {
     if (!c || !ms || bytes < 16 || iters == 0)
         return fail(LLM_E_ARG, "bad copy arguments");
+    c->busy = llm_ctx::WORK;
     HIP_TRY(hipSetDevice(c->device));
     const size_t n16 = bytes / 16;
     void *src = nullptr, *dst = nullptr;
@@ -2185,7 +2302,7 @@ std::string fmt_ms(double v) {
 
 // One forward of `rows` rows at `position` through layers [0, layer_count)
 // (run_composed_decoder_stack, host/host_qwen_8x64.cpp:1258-1445): the
-// rows (pinned host memory) into pair 1 by an asynchronous copy, Task 18
+// rows (pinned host memory) into pair 1 by a copy kernel, Task 18
 // (1 -> 0) and 19 (0 -> 1) per layer, Task 20 (1 -> 0) when `final_norm`.
 // Nothing is waited for, unless a line sink is set: then the forward is
 // bracketed by stream events per task, synchronised, and reported as the
@@ -2202,13 +2319,8 @@ int run_stack(llm_ctx_t* c, const int16_t* rows_host, uint32_t rows, uint32_t po
     auto enqueue = [&]() -> int {
         if (prof) HIP_TRY(hipEventRecord(c->gen_events[0], c->stream));
         invalidate_pair(c, 1);
-        if (rows == 1)  // a decode row: one contiguous copy (cheaper than a 2-D one)
-            HIP_TRY(hipMemcpyAsync(c->pairs[1], rows_host, (size_t)c->H * 2,
-                                   hipMemcpyHostToDevice, c->stream));
-        else
-            HIP_TRY(hipMemcpy2DAsync(c->pairs[1], (size_t)c->Hp * 2, rows_host,
-                                     (size_t)c->H * 2, (size_t)c->H * 2, rows,
-                                     hipMemcpyHostToDevice, c->stream));
+        HIP_TRY(llm::launch_io_rows(rows_host, c->H, c->pairs[1], c->Hp, c->H, rows, nullptr,
+                                    nullptr, 0, c->stream));
         c->n_h2d_rows++;
         if (prof) HIP_TRY(hipEventRecord(c->gen_events[1], c->stream));
         llm_status_t st;
@@ -2489,7 +2601,8 @@ int run_prompt_layers(llm_ctx* c, const int16_t* rows_host, uint32_t n, uint32_t
 }
 
 // The LM-head argmax of rows [row0, row0 + rows) of `pair` enqueued, its
-// keys copied into pinned host memory; the caller synchronises.
+// keys (which are 0 between argmaxes) published to pinned host memory as
+// transfer *seq.
 int ensure_keys_host(llm_ctx_t* c) {
     if (!c->keys_host &&
         hipHostMalloc((void**)&c->keys_host, 8 * sizeof(unsigned long long),
@@ -2498,13 +2611,13 @@ int ensure_keys_host(llm_ctx_t* c) {
     return 0;
 }
 
-int enqueue_argmax(llm_ctx_t* c, uint32_t pair, uint32_t row0, uint32_t rows) {
-    HIP_TRY(hipMemsetAsync(c->lm_keys, 0, 8 * sizeof(unsigned long long), c->stream));
+int enqueue_argmax(llm_ctx_t* c, uint32_t pair, uint32_t row0, uint32_t rows, uint32_t* seq) {
+    c->busy = llm_ctx::WORK;
     HIP_TRY(llm::launch_lm_argmax(c->lm.d, c->lm.steps, c->lm_vocab,
                                   c->pairs[pair] + (size_t)row0 * c->Hp, c->Hp, rows,
                                   c->lm.L, c->lm_keys, c->stream));
-    HIP_TRY(hipMemcpyAsync(c->keys_host, c->lm_keys, rows * sizeof(unsigned long long),
-                           hipMemcpyDeviceToHost, c->stream));
+    *seq = ++c->io_seq;
+    HIP_TRY(llm::launch_keys_out(c->lm_keys, c->keys_host, c->io_flag, *seq, c->stream));
     c->n_argmax++;
     return 0;
 }
@@ -2546,8 +2659,10 @@ int llm_lm_head_argmax(llm_ctx_t* c, uint32_t pair, uint32_t row0, uint32_t rows
     if (!c->lm_vocab) return fail(LLM_E_STATE, "LM head not loaded");
     HIP_TRY(hipSetDevice(c->device));
     if (int rc = ensure_keys_host(c)) return rc;
-    if (int rc = enqueue_argmax(c, pair, row0, rows)) return rc;
-    SYNC_TRY(c);
+    uint32_t seq;
+    if (int rc = enqueue_argmax(c, pair, row0, rows, &seq)) return rc;
+    if (int rc = io_wait(c, seq)) return rc;
+    if (int rc = check_waits(c)) return rc;
     for (uint32_t r = 0; r < rows; r++) {
         tokens[r] = key_token(c->keys_host[r]);
         if (scores) scores[r] = key_score(c->keys_host[r]);
@@ -2569,6 +2684,7 @@ int llm_generate(llm_ctx_t* c, const int16_t* embedding, uint32_t vocab,
         return fail(LLM_E_ARG, "sequence exceeds max_seq_len");
     for (uint32_t t = 0; t < n_prompt; t++)
         if (prompt[t] >= vocab) return fail(LLM_E_ARG, "prompt token outside the vocabulary");
+    c->busy = llm_ctx::WORK;
     HIP_TRY(hipSetDevice(c->device));
     llm_generate_stats_t local{};
     llm_generate_stats_t& S = stats ? *stats : local;
@@ -2591,11 +2707,14 @@ int llm_generate(llm_ctx_t* c, const int16_t* embedding, uint32_t vocab,
         c->stage_rows = need;
     }
     if (int rc = ensure_keys_host(c)) return rc;
-    if (int rc = gen_events(c, 2 + 2 * (size_t)layer_count + 1 + 5)) return rc;
+    if (int rc = gen_events(c, 2 + 2 * (size_t)layer_count + 1 + 8)) return rc;
     const size_t ne = c->gen_events.size();
-    hipEvent_t ev_p0 = c->gen_events[ne - 5], ev_p1 = c->gen_events[ne - 4],
-               ev_a = c->gen_events[ne - 3], ev_b = c->gen_events[ne - 2],
-               ev_l = c->gen_events[ne - 1];
+    hipEvent_t ev_p0 = c->gen_events[ne - 8], ev_p1 = c->gen_events[ne - 7];
+    // before a forward's rows' copy, after its last task, after its argmax:
+    // two sets, so that a step's times are read behind the next forward
+    hipEvent_t* ev_a = &c->gen_events[ne - 6];
+    hipEvent_t* ev_b = &c->gen_events[ne - 4];
+    hipEvent_t* ev_l = &c->gen_events[ne - 2];
     for (uint32_t t = 0; t < n_prompt; t++)
         std::memcpy(c->stage + (size_t)t * c->H, embedding + (size_t)prompt[t] * c->H,
                     (size_t)c->H * 2);
@@ -2645,8 +2764,13 @@ int llm_generate(llm_ctx_t* c, const int16_t* embedding, uint32_t vocab,
     // up: what was enqueued since the previous one (`redo`) runs again, once,
     // on launches without such waits, and is synchronised.  K/V rows of the
     // invalid run are rewritten by the re-run from the same inputs.
+    uint32_t seq = 0;  // transfer of the last argmax's keys
     auto settle = [&](const std::function<int()>& redo) -> int {
-        HIP_TRY(hipStreamSynchronize(c->stream));
+        if (seq) {
+            if (int r = io_wait(c, seq)) return r;
+        } else {
+            HIP_TRY(hipStreamSynchronize(c->stream));
+        }
         if (!clear_waits(c)) return 0;
         WaitFreeScope wf(c);
         c->n_wait_reruns++;
@@ -2661,58 +2785,58 @@ int llm_generate(llm_ctx_t* c, const int16_t* embedding, uint32_t vocab,
     }
     // sampled tokens (host/host_qwen_8x64.cpp:9091-9136); times from stream
     // events: a forward from before its rows' copy to after its last task,
-    // the LM head from there to its keys' copy
+    // the LM head from there to its keys' transfer
+    auto times = [&](uint32_t step) -> int {
+        const uint32_t e = step & 1;
+        HIP_TRY(hipEventSynchronize(ev_l[e]));
+        if (step == 0) {
+            S.prompt_forward_ms = event_ms(ev_p0, ev_p1);
+            S.lm_head_ms += event_ms(ev_p1, ev_l[e]);
+        } else {
+            S.generated_forward_ms += event_ms(ev_a[e], ev_b[e]);
+            S.lm_head_ms += event_ms(ev_b[e], ev_l[e]);
+        }
+        return 0;
+    };
+    auto forward = [&](uint32_t step, uint32_t* tasks) -> int {  // of the token sampled before it
+        const uint32_t t = n_prompt + step - 1;
+        HIP_TRY(hipEventRecord(ev_a[step & 1], c->stream));
+        if (int r = run_stack(c, c->stage + (size_t)t * c->H, 1, t, layer_count, true, false, tasks))
+            return r;
+        HIP_TRY(hipEventRecord(ev_b[step & 1], c->stream));
+        return 0;
+    };
     auto gen0 = std::chrono::steady_clock::now();
     uint32_t token = 0;
     for (uint32_t step = 0; step < max_new_tokens; step++) {
         auto argmax = [&]() -> int {
-            if (int r = enqueue_argmax(c, 0, last_row, 1)) return r;
-            HIP_TRY(hipEventRecord(ev_l, c->stream));
+            if (int r = enqueue_argmax(c, 0, last_row, 1, &seq)) return r;
+            HIP_TRY(hipEventRecord(ev_l[step & 1], c->stream));
             return 0;
         };
         if ((rc = argmax())) return rc;
-        if (step == 0) {
-            rc = settle([&] {
-                const int r = run_prompt(false);
-                return r ? r : argmax();
-            });
-        } else {
-            const uint32_t prev = n_prompt + step - 1;  // the last forward's row
-            rc = settle([&]() -> int {
-                uint32_t uncounted = 0;
-                HIP_TRY(hipEventRecord(ev_a, c->stream));
-                if (int r = run_stack(c, c->stage + (size_t)prev * c->H, 1, prev, layer_count,
-                                      true, false, &uncounted))
-                    return r;
-                HIP_TRY(hipEventRecord(ev_b, c->stream));
-                return argmax();
-            });
-        }
+        rc = settle([&]() -> int {
+            uint32_t uncounted = 0;
+            const int r = step == 0 ? run_prompt(false) : forward(step, &uncounted);
+            return r ? r : argmax();
+        });
         if (rc) return rc;
         token = key_token(c->keys_host[0]);
         if (step == 0) {
-            S.prompt_forward_ms = event_ms(ev_p0, ev_p1);
-            S.lm_head_ms += event_ms(ev_p1, ev_l);
             S.time_to_first_token_ms = ms_since(begin);
             gen0 = std::chrono::steady_clock::now();  // the generated forwards from here
-        } else {
-            S.generated_forward_ms += event_ms(ev_a, ev_b);
-            S.lm_head_ms += event_ms(ev_b, ev_l);
         }
         out_tokens[step] = token;
         if (step + 1 < max_new_tokens) {
             if (token >= vocab) return fail(LLM_E_STATE, "sampled token outside the embedding");
-            int16_t* row = c->stage + ((size_t)n_prompt + step) * c->H;
-            std::memcpy(row, embedding + (size_t)token * c->H, (size_t)c->H * 2);
-            HIP_TRY(hipEventRecord(ev_a, c->stream));
-            if ((rc = run_stack(c, row, 1, n_prompt + step, layer_count, true, false,
-                                &S.coarse_task_count)))
-                return rc;
-            HIP_TRY(hipEventRecord(ev_b, c->stream));
+            std::memcpy(c->stage + ((size_t)n_prompt + step) * c->H,
+                        embedding + (size_t)token * c->H, (size_t)c->H * 2);
+            if ((rc = forward(step + 1, &S.coarse_task_count))) return rc;
             S.generated_forward_passes++;
             S.output_materializations++;
             last_row = 0;
         }
+        if ((rc = times(step))) return rc;
     }
     S.generated_wall_ms = max_new_tokens > 1 ? ms_since(gen0) : 0.0;
     S.total_ms = ms_since(begin);

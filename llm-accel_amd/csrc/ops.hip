@@ -252,8 +252,8 @@ __global__ __launch_bounds__(256) void op_flash_kernel(OpFlashArgs a) {
 // the running maximum is a maximum, so it needs no sequence -- the tile's
 // probabilities, sum and PV values, (3) the sequential rescale of sums and
 // values, one addition per tile except where the maximum rises.  The walk
-// above takes ~5 us per tile; these three launches ~4 us each at 24 tiles
-// (128 query rows: 125 -> 15 us).  K and V are staged clamped in LDS, in
+// above takes ~5 us per tile; these three launches 7.5, 6.4 and 4.6 us at 8
+// tiles and 128 query rows (48 -> 18 us), little more at 24 (125 -> ~20).  K and V are staged clamped in LDS, in
 // the pages' bank-paired order (attn_common.h).
 // ---------------------------------------------------------------------
 struct OpTile {
@@ -490,7 +490,7 @@ hipError_t launch_op_flash(const OpFlashArgs& a, hipStream_t st) {
     if (a.kv_heads * a.tokens * a.group == 0 || a.head_dim == 0 || a.head_dim > 128 ||
         a.head_dim % 16 != 0 || a.pos0 + a.tokens > a.tiles * 64)
         return hipErrorInvalidValue;
-    // the three launches (~13 us) from the tiles whose walk takes longer
+    // the three launches from the tiles whose walk takes as long (~5 us each)
     const uint32_t nt = (a.pos0 + a.tokens + 63) / 64;
     if (nt >= 3 && a.group <= 16 && a.tokens <= 8) {
         const uint32_t grid = a.tokens * a.kv_heads * nt;

@@ -384,9 +384,10 @@ class Accelerator:
         self._check(rc, "llm_op")
         if not sync:
             return None, st
-        self.sync()
-        out = self.port_read(PORT_OUT, out_elems) if out_elems else None
-        return out, st
+        if not out_elems:
+            self.sync()
+            return None, st
+        return self.port_read(PORT_OUT, out_elems), st  # waits for the operator
 
     def _checked(self, op, st):
         if st.code != STATUS_OK:
