@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -42,18 +43,37 @@ __device__ __forceinline__ uint32_t plane_d(uint32_t w0, uint32_t w1) {
 // every sum exact in int32 (K <= 16384).  Byte-plane weights (16-bit
 // matrices) are w = 256 a + b + 128, which adds 128 sum x.
 //
-// Four wavefronts per workgroup, 2 x 2 over 64 MT rows x 128 outputs (64
-// outputs of gate and of up for EPI_SILU); the MFMA's A operand is the
-// weights, so a lane's results are runs of 4 outputs of one row.  Per
-// 128-input step the weights go through LDS, unpacked once per workgroup
-// (double-buffered, one barrier per step, the step after next already in
-// flight); the activation planes are in operand order and come straight
-// from L2, each 32-input piece reloaded right after its last use.
+// Wavefronts 2 WM: each 32 rows x 64 output slots (32 outputs of gate and of
+// up for EPI_SILU), two over 128 slots, WM over the row pieces; the MFMA's A
+// operand is the weights, so a lane's results are runs of 4 outputs of one
+// row.  Per 128-input step the weights go through LDS, unpacked once per
+// workgroup (double-buffered, one barrier per step, two more steps in
+// flight); the activation planes are in operand order and come straight from
+// L2, each 32-input piece reloaded for the next step after its last use.
+// With four row pieces a workgroup fills a compute unit (two wavefronts per
+// SIMD) and takes its items in turn, the next item's loads already under way
+// during an item's epilogue.  1,024 rows of config B: gate|up 189 us (369 G
+// i8 operations, 2.0 POPS; one item per workgroup 213), Q|K|V 31, O 30, down
+// 90 with K in two parts.  A plain loop of these products runs at 3.4 POPS on
+// such data (the card's power limit; 4.3 on constant data), so gate|up is
+// bounded by 110 us: what is left is the unpacking and epilogue arithmetic
+// that shares the SIMDs and the uneven last round (5.4 items per workgroup).
+// Measured and not kept: 64 x 64 per wavefront (one per SIMD: 299 us), the
+// activations requested two steps ahead (no change), a raised wave priority
+// around the products (194 us).  Kernels stay small: with the corrections in
+// every variant (40 KB of code) a launch began ~20 us later.
 // ---------------------------------------------------------------------
 constexpr uint32_t kWHalf = 544, kWPlane = 2 * kWHalf, kWPiece = 2368;  // LDS strides (padded)
+constexpr uint32_t kPfItems = 16;  // of a workgroup
 constexpr uint32_t kWBuf = 16 * kWPiece;  // [4 n pieces][4 k pieces]
 static_assert(kWPiece >= 2 * kWPlane && kWPiece % 16 == 0, "piece holds two planes");
 
+template <typename T>
+__device__ __forceinline__ void swap_v(T& a, T& b) {
+    const T t = a;
+    a = b;
+    b = t;
+}
 // b = the low byte, a = h - 8 + (l >> 7): w + 2048 = 256 h + l.
 __device__ __forceinline__ uint32_t p12_signed_high(uint32_t h4, uint32_t l4) {
     const uint32_t t = h4 + ((l4 >> 7) & 0x01010101u);
@@ -84,38 +104,38 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
                                                               uint32_t ntiles) {
     constexpr bool SILU = EPI == EPI_SILU;
     constexpr int NTH = 128 * WM, NP = 1024 / NTH;  // threads, weight pieces per thread
+    constexpr uint32_t ITEMS = WM == 4 ? kPfItems : 1;
     __shared__ __attribute__((aligned(16))) uint8_t wl[2 * kWBuf];
-    __shared__ int32_t sw[128], swl[128];  // a slot's weight sum: s, or as pf_narrow12 takes it
-    __shared__ int32_t gg[EPI == EPI_RESID ? 128 : 1];
+    __shared__ int2 sw[ITEMS][128];  // per item a slot's weight sum, as pf_narrow12 takes it
+    __shared__ int32_t gg[EPI == EPI_RESID ? ITEMS : 1][EPI == EPI_RESID ? 128 : 1];
     __shared__ uint32_t silu[SILU ? 2049 : 1];
     __shared__ uint32_t last;
-    // the row tiles of one output tile run on one XCD (workgroups go round
-    // the 8 XCDs), which then reads the tile's weights from HBM once
-    const uint32_t parts = a.parts;
-    uint32_t j = blockIdx.x >> 3;
-    const uint32_t mi = j % mtiles;
-    j /= mtiles;
-    const uint32_t part = j % parts, ni = (j / parts) * 8 + (blockIdx.x & 7);
-    if (ni >= ntiles) return;
+    // Items (row tile, part of K, output tile) of this workgroup: the items
+    // of one output tile run on one XCD (workgroups go round the 8 XCDs),
+    // which then reads the tile's weights from HBM once; item j0 + i stride.
+    const uint32_t parts = a.parts, xcd = blockIdx.x & 7;
+    const uint32_t j0 = blockIdx.x >> 3, stride = gridDim.x >> 3;
+    const uint32_t njx = xcd < ntiles ? ((ntiles - xcd + 7) / 8) * parts * mtiles : 0;
+    if (j0 >= njx) return;
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave >> 1, wn = wave & 1, half = lane >> 5;
     const uint32_t S = a.steps, KC = 4 * S;
-    const uint32_t s0 = part * S / parts, s1 = (part + 1) * S / parts;
-    // output and matrix of slot i (0..127) of the workgroup's n pieces
-    auto slot_n = [&](uint32_t i) {
+    auto item_n = [&](uint32_t j) { return j / mtiles / parts * 8 + xcd; };  // output tile
+    auto item_part = [&](uint32_t j) { return j / mtiles % parts; };
+    // output and matrix of slot i (0..127) of output tile ni
+    auto slot_n = [&](uint32_t ni, uint32_t i) {
         return SILU ? ni * 64 + 32 * (i >> 6) + (i & 31) : ni * 128 + i;
     };
     auto slot_m = [&](uint32_t i) { return SILU ? (i >> 5) & 1 : 0u; };
-    if (tid < 128) {
-        const uint32_t n = slot_n(tid);
-        const int32_t* ms = SILU && slot_m(tid) ? a.ms1 : a.ms0;
+    for (uint32_t i = tid >> 7; i < ITEMS && j0 + i * stride < njx; i += (NTH + 127) / 128) {
+        const uint32_t sl = tid & 127, n = slot_n(item_n(j0 + i * stride), sl);
+        const int32_t* ms = SILU && slot_m(sl) ? a.ms1 : a.ms0;
         const bool ok = n < a.n;
         const int32_t sum = ok ? 256 * ms[2 * n] + ms[2 * n + 1] + (WIDE ? 0 : 128 * 64 * (int32_t)a.kq) : 0;
-        sw[tid] = WIDE ? sum : (sum >> 1) + 8;
-        swl[tid] = 128 * (sum & 1) + 8;
+        sw[i][sl] = WIDE ? make_int2(sum, 0) : make_int2((sum >> 1) + 8, 128 * (sum & 1) + 8);
         if (EPI == EPI_RESID)
-            gg[tid] = ok && a.xp_out ? __mul24(a.norm_gain, (int32_t)a.norm_gamma[n]) : 0;
+            gg[i][sl] = ok && a.xp_out ? __mul24(a.norm_gain, (int32_t)a.norm_gamma[n]) : 0;
     }
     if (SILU)
         for (uint32_t i = tid; i < 2049; i += NTH) silu[i] = a.silu8[i];
@@ -126,18 +146,23 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
     uint32_t woff[NP], wdst[NP];
 #pragma unroll
     for (int q = 0; q < NP; q++) {
-        const uint32_t slot = (NTH / 8) * q + (tid >> 3), n = slot_n(slot);
+        const uint32_t slot = (NTH / 8) * q + (tid >> 3);
         const bool up = SILU && __builtin_amdgcn_readfirstlane(slot_m(slot));
-        if (WIDE) {
-            wbase[q] = (const uint8_t*)(up ? a.mf1 : a.mf0);
-            woff[q] = min(n / kMfRows, (a.n - 1) / kMfRows) * a.kq * kMfRecord +
-                      (16 * (pc & 3) + n % kMfRows) * 16;
-        } else {
-            wbase[q] = up ? a.p1 : a.p0;
-            woff[q] = min(n >> 2, (a.n + 3) / 4 - 1) * S * kP12Step + 128 * (n & 3) + 16 * pc;
-        }
+        wbase[q] = WIDE ? (const uint8_t*)(up ? a.mf1 : a.mf0) : (up ? a.p1 : a.p0);
         wdst[q] = (4 * (slot >> 5) + (pc >> 1)) * kWPiece + (pc & 1) * kWHalf + 16 * (slot & 31);
     }
+    auto w_item = [&](uint32_t j) {  // the pieces' offsets in item j's output tile
+        const uint32_t ni = item_n(j);
+#pragma unroll
+        for (int q = 0; q < NP; q++) {
+            const uint32_t n = slot_n(ni, (NTH / 8) * q + (tid >> 3));
+            if (WIDE)
+                woff[q] = min(n / kMfRows, (a.n - 1) / kMfRows) * a.kq * kMfRecord +
+                          (16 * (pc & 3) + n % kMfRows) * 16;
+            else
+                woff[q] = min(n >> 2, (a.n + 3) / 4 - 1) * S * kP12Step + 128 * (n & 3) + 16 * pc;
+        }
+    };
     const uint32_t noff = 512 - 64 * ((tid >> 3) & 3) - 8 * pc;  // to a piece's high nibbles
     v4u wr[2][NP];
     v4u wr2[WIDE ? 2 : 1][WIDE ? NP : 1];
@@ -159,10 +184,11 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
             }
         }
     };
-    auto w_store = [&](int set) {  // into buffer `set`
+    uint32_t flip = 0;  // buffer of register set 0
+    auto w_store = [&](int set) {
 #pragma unroll
         for (int q = 0; q < NP; q++) {
-            uint8_t* d = wl + set * kWBuf + wdst[q];
+            uint8_t* d = wl + (set ^ flip) * kWBuf + wdst[q];
             if constexpr (WIDE) {
                 *(v4u*)d = wr[set][q];
                 *(v4u*)(d + kWPlane) = wr2[set][q];
@@ -182,30 +208,51 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
             }
         }
     };
-    const uint32_t mp = mi * WM + wm;  // this wavefront's row piece
-    const int8_t* xs = a.x + (size_t)mp * KC * 2048;
-    v4i xb[2][4][2];
-    auto x_load = [&](int set, int kc, uint32_t k) {
+    v4i xb[4][2];
+    // Cursors over the items' steps, the weights' and the activations' each
+    // ahead of the products'; past the last step they repeat it.
+    struct Cursor {
+        uint32_t j, s, end;
+    };
+    auto first_step = [&](uint32_t j) { return item_part(j) * S / parts; };
+    auto last_step = [&](uint32_t j) { return (item_part(j) + 1) * S / parts; };
+    Cursor cw = {j0, first_step(j0), last_step(j0)}, cx = cw;
+    const int8_t* xs = nullptr;
+    auto x_item = [&](uint32_t j) { xs = a.x + (size_t)(j % mtiles * WM + wm) * KC * 2048; };
+    auto advance = [&](Cursor& c) {  // whether it entered another item
+        if (++c.s < c.end) return false;
+        if (c.j + stride >= njx) {
+            c.s--;
+            return false;
+        }
+        c.j += stride;
+        c.s = first_step(c.j);
+        c.end = last_step(c.j);
+        return true;
+    };
+    auto w_next = [&](int set) {
+        w_load(set, cw.s);
+        if (advance(cw)) w_item(cw.j);
+    };
+    auto x_load = [&](int kc) {
 #pragma unroll
         for (int p = 0; p < 2; p++)
-            xb[set][kc][p] = *(const v4i*)(xs + (size_t)k * 2048 + 1024 * p + lane * 16);
+            xb[kc][p] =
+                *(const v4i*)(xs + (size_t)(4 * cx.s + kc) * 2048 + 1024 * p + lane * 16);
+    };
+    auto x_next = [&] {
+        if (advance(cx)) x_item(cx.j);
     };
     v16i acc[2][3];
+    w_item(j0);
+    x_item(j0);
+    w_next(0);
+    w_next(1);
 #pragma unroll
-    for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-        for (int p = 0; p < 3; p++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[nt][p][i] = 0;
-    auto clamp_s = [&](uint32_t s) { return s < s1 ? s : s1 - 1; };
-    w_load(0, s0);
-    w_load(1, clamp_s(s0 + 1));
-#pragma unroll
-    for (int kc = 0; kc < 4; kc++) x_load(0, kc, 4 * s0 + kc);
-#pragma unroll
-    for (int kc = 0; kc < 4; kc++) x_load(1, kc, 4 * clamp_s(s0 + 1) + kc);
+    for (int kc = 0; kc < 4; kc++) x_load(kc);
+    x_next();
     w_store(0);
-    w_load(0, clamp_s(s0 + 2));
+    w_next(0);
     lds_barrier();
     // weight operands of piece kc of buffer b
     const uint32_t rd = 2 * wn * 4 * kWPiece + (lane & 31) * 16 + half * kWHalf;
@@ -215,55 +262,71 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
         for (int nt = 0; nt < 2; nt++)
 #pragma unroll
             for (int p = 0; p < 2; p++)
-                wf[set][nt][p] =
-                    *(const v4i*)(wl + b * kWBuf + rd + (4 * nt + kc) * kWPiece + p * kWPlane);
+                wf[set][nt][p] = *(const v4i*)(wl + (b ^ flip) * kWBuf + rd +
+                                               (4 * nt + kc) * kWPiece + p * kWPlane);
     };
     wf_load(0, 0, 0);
-    // Step s from buffer P.  Piece kc's operands were read before the
+    // A step from register sets and buffer P.  Piece kc's operands were read before the
     // products of the piece before it; the next step's weights go into the
     // other buffer in the middle (its last readers passed the barrier of
     // the step before), so that the barrier, before the last piece, leaves
     // products to issue behind it.  A piece's activations are reloaded for
-    // the step after next once used and the weights three steps on requested:
-    // a wavefront's loads complete in order, so that activations requested
-    // only one step ahead wait for the weights (HBM) requested before them
-    // (measured 1.5 us a step against 1.0 us of products).
-    auto step = [&](auto par, uint32_t s) {
+    // the next step once used, the weights three steps on requested.
+    auto step = [&](auto par) {
         constexpr int P = decltype(par)::value;
-        const uint32_t k2 = 4 * clamp_s(s + 2);
 #pragma unroll
         for (int kc = 0; kc < 4; kc++) {
             const int cur = kc & 1;
             if (kc < 3) wf_load(cur ^ 1, P, kc + 1);
             else wf_load(cur ^ 1, P ^ 1, 0);
             if (kc == 1) w_store(P ^ 1);
-            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int nt = 0; nt < 2; nt++) {
                 v16i* c = acc[nt];
-                const v4i *w = wf[cur][nt], *x = xb[P][kc];
+                const v4i *w = wf[cur][nt], *x = xb[kc];
                 c[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[0], x[0], c[0], 0, 0, 0);
                 c[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[0], x[1], c[1], 0, 0, 0);
                 c[2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[1], x[1], c[2], 0, 0, 0);
                 c[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[1], x[0], c[1], 0, 0, 0);
             }
-            __builtin_amdgcn_s_setprio(0);
-            x_load(P, kc, k2 + kc);
-            if (kc == 1) w_load(P ^ 1, clamp_s(s + 3));
+            x_load(kc);
+            if (kc == 1) w_next(P ^ 1);
+            if (kc == 3) x_next();
             // keeps each piece's loads where they are: gathered at the end of
             // the step they have no products left to hide behind
             __builtin_amdgcn_sched_barrier(0);
             if (kc == 2) lds_barrier();
         }
     };
-    for (uint32_t s = s0; s < s1; s += 2) {
-        step(std::integral_constant<int, 0>{}, s);
-        if (s + 1 < s1) step(std::integral_constant<int, 1>{}, s + 1);
+    for (uint32_t j = j0, it = 0; j < njx; j += stride, it++) {
+    const uint32_t ni = item_n(j), part = item_part(j);
+    const uint32_t mp = j % mtiles * WM + wm;  // this wavefront's row piece
+    const uint32_t len = last_step(j) - first_step(j);
+#pragma unroll
+    for (int nt = 0; nt < 2; nt++)
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[nt][p][i] = 0;
+    for (uint32_t s = 0; s + 1 < len; s += 2) {
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+    }
+    if (len & 1) {
+        // the sets change places
+        step(std::integral_constant<int, 0>{});
+        flip ^= 1;
+#pragma unroll
+        for (int q = 0; q < NP; q++) {
+            swap_v(wr[0][q], wr[1][q]);
+            if constexpr (WIDE) swap_v(wr2[0][q], wr2[1][q]);
+            else swap_v(wn8[0][q], wn8[1][q]);
+        }
     }
     if (parts > 1) {
         // exact sums of this part; the last of the tile's parts to arrive
         // adds the others'
-        const size_t tile = (size_t)ni * mtiles + mi;
+        const size_t tile = (size_t)ni * mtiles + j % mtiles;
         int64_t* base = a.part + tile * parts * (size_t)(NTH * 32) + tid;
         int64_t t[32];
 #pragma unroll
@@ -272,7 +335,7 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
             t[i] = ((((int64_t)c[0][i & 15] << 8) + c[1][i & 15]) << 8) + c[2][i & 15];
             st_coherent(base + ((size_t)part * 32 + i) * NTH, t[i]);
         }
-        if (!arrive_last(&a.count[tile], parts, &last)) return;
+        if (!arrive_last(&a.count[tile], parts, &last)) continue;
 #pragma unroll 1
         for (uint32_t q = 1; q < parts; q++) {
             const int64_t* o = base + (size_t)((part + q) % parts) * 32 * NTH;
@@ -301,11 +364,11 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
             const int32_t ac = acc[nt][0][i], x = acc[nt][1][i], bd = acc[nt][2][i];
             if (WIDE)
                 return pf_narrow64(65536 * (int64_t)ac + 256 * (int64_t)x + bd +
-                                   128 * ((int64_t)sw[slot] + rx));
-            int32_t sh = sw[slot], sl = swl[slot];
-            if (CORR && corr && slot_n(slot) < a.n) {
+                                   128 * ((int64_t)sw[it][slot].x + rx));
+            int32_t sh = sw[it][slot].x, sl = sw[it][slot].y;
+            if (CORR && corr && slot_n(ni, slot) < a.n) {
                 // corrections of weights past 12 bits: x from its planes
-                const uint4 cw = *(const uint4*)(corr + (size_t)kCorrSlots * slot_n(slot));
+                const uint4 cw = *(const uint4*)(corr + (size_t)kCorrSlots * slot_n(ni, slot));
                 const uint32_t e[4] = {cw.x, cw.y, cw.z, cw.w};
                 int64_t more = 0;
 #pragma unroll
@@ -343,16 +406,26 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
             }
         };
         if constexpr (SILU) {
-            int32_t y[16];
+            // in three passes, each over all 16 outputs: the sums narrowed
+            // (which frees their registers), the table words, the products
+            int32_t gate[16], up[16], y[16];
+            uint32_t tw[16];
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const uint32_t r = 8 * (i >> 2) + 4 * half + (i & 3);
-                const uint32_t sg = 64 * wn + r;
-                const int32_t gate = value(0, i, sg, a.corr0);
-                const int32_t up = value(1, i, sg + 32, a.corr1);
-                const int32_t sv = silu_packed(gate, silu[fx_silu_index(gate)]);
-                y[i] = med3((__mul24(sv, up) + 128) >> 8, INT16_MIN, INT16_MAX);
-                if (slot_n(sg) >= a.n) y[i] = 0;
+                const uint32_t sg = 64 * wn + 8 * (i >> 2) + 4 * half + (i & 3);
+                gate[i] = value(0, i, sg, a.corr0);
+                up[i] = value(1, i, sg + 32, a.corr1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 16; i++) tw[i] = silu[fx_silu_index(gate[i])];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const uint32_t sg = 64 * wn + 8 * (i >> 2) + 4 * half + (i & 3);
+                const int32_t sv = silu_packed(gate[i], tw[i]);
+                y[i] = med3((__mul24(sv, up[i]) + 128) >> 8, INT16_MIN, INT16_MAX);
+                if (slot_n(ni, sg) >= a.n) y[i] = 0;
             }
             store_xp(y, ni * 2 + wn, 2 * ntiles);
         } else {
@@ -383,11 +456,12 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
                 if (EPI == EPI_RESID && a.xp_out) {
 #pragma unroll
                     for (int i = 0; i < 16; i++)
-                        y[i] = norm1(y[i], gg[sl + 8 * (i >> 2) + 4 * half + (i & 3)]);
+                        y[i] = norm1(y[i], gg[it][sl + 8 * (i >> 2) + 4 * half + (i & 3)]);
                     store_xp(y, ni * 4 + 2 * wn + nt, 4 * ntiles);
                 }
             }
         }
+    }
     }
 }
 
@@ -911,7 +985,15 @@ __device__ __forceinline__ void pf_attention_body(const PfAttnArgs& a, PfAttnSme
             sum[rt] = __builtin_elementwise_add_sat(rnd16_mul(sum[rt], old[rt]), tsum);
         }
         // ---- PV of strips w, w + 4: element 16 strip + 4 g + s ----
-        const bool rise = __any(old[0] != 65536 || old[1] != 65536);
+        if (__any(old[0] != 65536 || old[1] != 65536)) {  // else the factors are 1.0
+#pragma unroll
+            for (int es = 0; es < ES; es++)
+#pragma unroll
+                for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+                    for (int s = 0; s < 4; s++)
+                        acc[es][rt][s] = rnd16_mul(acc[es][rt][s], old[rt]);
+        }
 #pragma unroll
         for (int es = 0; es < ES; es++) {
 #pragma unroll
@@ -932,9 +1014,7 @@ __device__ __forceinline__ void pf_attention_body(const PfAttnArgs& a, PfAttnSme
                                          (uint32_t)bd[s];
                     // rnd(rnd(tot, 6), 8) = floor((tot + 2^5 + 2^13) / 2^14)
                     const int32_t tv = med3((int32_t)(tot + 8224) >> 14, INT16_MIN, INT16_MAX);
-                    int32_t v = acc[es][rt][s];
-                    if (rise) v = rnd16_mul(v, old[rt]);
-                    acc[es][rt][s] = __builtin_elementwise_add_sat(v, tv << 8);
+                    acc[es][rt][s] = __builtin_elementwise_add_sat(acc[es][rt][s], tv << 8);
                 }
             }
         }
@@ -977,8 +1057,12 @@ __global__ __launch_bounds__(256, 2) void pf_attention_kernel(PfAttnArgs a) {
 template <int WM, int EPI>
 hipError_t pf_gemm(const PfGemmArgs& a, uint32_t ntiles, hipStream_t st) {
     const uint32_t mtiles = (a.m + 32 * WM - 1) / (32 * WM);
-    const uint32_t grid = 8 * mtiles * a.parts * ((ntiles + 7) / 8);
-    const dim3 g(grid), b(128 * WM);
+    // items of the fullest XCD; a workgroup of four row pieces, one per
+    // compute unit, takes several in turn (at most kPfItems)
+    const uint32_t items = mtiles * a.parts * ((ntiles + 7) / 8);
+    uint32_t wgs = items;
+    if (WM == 4) wgs = std::max(std::min(items, 32u), (items + kPfItems - 1) / kPfItems);
+    const dim3 g(8 * wgs), b(128 * WM);
     if (!a.p0)
         hipLaunchKernelGGL((pf_gemm_kernel<WM, EPI, true, false>), g, b, 0, st, a, mtiles, ntiles);
     else if (a.corr0 || a.corr1)
@@ -1002,7 +1086,7 @@ hipError_t pf_gemm_w(const PfGemmArgs& a, uint32_t ntiles, uint32_t wm, hipStrea
 // Row pieces per workgroup: the fewest that hold the rows, at most four (the
 // weights of a workgroup are unpacked once for all of them).  K is split
 // while the tiles alone leave half of the 256 compute units idle: the parts'
-// exchange takes ~15 us on a full chip, a 128-input step 1.5 us, so at least
+// exchange takes ~15 us on a full chip, a 128-input step ~1.5 us, so at least
 // 32 steps stay with a part there (down, 1,024 rows, 86 steps: 137 us whole,
 // 85 in two parts; Q|K|V, 16 steps: 33 and 47) and 8 where it is nearly
 // empty (16 rows, down: 122 us whole, 31 in eight parts; O: 28 and 22).
