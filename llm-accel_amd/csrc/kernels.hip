@@ -1197,8 +1197,12 @@ static hipError_t launch_lm_rt(const int16_t* w, uint32_t steps, uint32_t n,
                                const int16_t* x, uint32_t ldx, uint32_t rows, int L,
                                unsigned long long* keys, hipStream_t st) {
     const uint32_t nblocks = (n + 3) / 4;
+    // Every workgroup ends with one atomicMax on the same line: 384 of them,
+    // three per two compute units, not one per four blocks (16,384 rows of
+    // 2,048 / 896: call 29.3 / 23.1 us with up to 2,048 workgroups, 21.9 /
+    // 16.6 with 384, 24.0 / 17.9 with 512; 151,936 rows of 2,048 115 -> 109).
     uint32_t grid = (nblocks + 3) / 4;
-    if (grid > 2048) grid = 2048;
+    if (grid > 384) grid = 384;
     if (RT <= 2 && steps <= kLmStageSteps) {
         constexpr bool XS = RT <= 2;
         switch (L) {
@@ -1226,15 +1230,17 @@ hipError_t launch_lm_argmax(const int16_t* w, uint32_t steps, uint32_t n,
     // From three rows on the matrix cores (call times at hidden 2048, 151,936
     // rows: 3 rows 236 -> 135 us, 5 410 -> 135, 8 415 -> 134; one and two
     // rows 122 and 128 us against 134).  Tables of fewer groups than 2,048
-    // wavefronts can walk share each among a workgroup's wavefronts; larger
-    // ones take one workgroup per compute unit (512 and 1,024 workgroups:
-    // 153 and 139 us, their last round nearly empty).
+    // wavefronts can walk share each among a workgroup's wavefronts, at most
+    // 512 of them (their final atomics share a line: 30,000 rows of 2,048 in
+    // 38 us, 49 with a workgroup per group); larger ones take one workgroup
+    // per compute unit (512 and 1,024 workgroups: 153 and 139 us, their last
+    // round nearly empty).
     const uint32_t groups = (n + kLmGroup - 1) / kLmGroup;
     const bool shared = groups < 2048;
     if (rows >= 3 && steps <= (shared ? kLmMfmaStepsShared : kLmMfmaSteps)) {
         const uint32_t lds = steps * 2048;
         if (shared)
-            lm_argmax_mfma_kernel<true><<<groups, 256, lds, st>>>(w, steps, n, x, ldx, rows, keys);
+            lm_argmax_mfma_kernel<true><<<std::min(groups, 512u), 256, lds, st>>>(w, steps, n, x, ldx, rows, keys);
         else
             lm_argmax_mfma_kernel<false><<<256, 256, lds, st>>>(w, steps, n, x, ldx, rows, keys);
         return hipGetLastError();
