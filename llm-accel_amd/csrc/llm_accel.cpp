@@ -1826,7 +1826,13 @@ int enqueue_op_projection(llm_ctx* c, uint32_t layer, uint32_t proj, uint32_t T,
     const uint32_t row0 = proj == 1 ? c->H : proj == 2 ? c->H + c->Ckv : 0;
     const uint32_t n = proj == 0 ? c->H : (proj <= 2 ? c->Ckv : m.n);
     if (T == 0) return 0;
-    if (m.k % 8 == 0 && (uintptr_t)in % 16 == 0)  // what the copy kernel's loads need
+    // the kernels read whole k-steps and, for 3 rows on, all 8 rows: the
+    // context's own port holds those where its tight rows are whole steps;
+    // otherwise the rows are staged
+    const bool direct = in == c->ports[LLM_PORT_IN] && m.k == m.k_pad &&
+                        (out + (size_t)T * n <= in || out >= in + c->port_n);
+    if (direct) {
+    } else if (m.k % 8 == 0 && (uintptr_t)in % 16 == 0)  // what the copy kernel's loads need
         HIP_TRY(llm::launch_io_rows(in, m.k, c->op_stage, m.k_pad, m.k, T, nullptr, nullptr, 0,
                                     c->stream));
     else
@@ -1835,7 +1841,7 @@ int enqueue_op_projection(llm_ctx* c, uint32_t layer, uint32_t proj, uint32_t T,
     llm::ProjArgs a{};
     a.w0 = m.d ? m.d + (size_t)row0 * m.k_pad : nullptr;
     a.steps = m.steps;
-    a.x = c->op_stage;
+    a.x = direct ? in : c->op_stage;
     a.ldx = m.k_pad;
     a.out = out;
     a.ldo = n;
