@@ -122,6 +122,22 @@ def test_long_prompt(monkeypatch):
     _compare(monkeypatch, D128, "plain", 1100, 8)
 
 
+# Shapes whose products have more tiles than workgroups, which then take several in
+# turn: gate|up with one and three 128-input steps per tile (even and odd numbers of
+# steps leave the buffers' parity either way), and down with K in four parts.
+TURN1 = workloads.ShapeSpec("turn1", 512, 128, 6016, 1, 4, 2, 1200, 0.25, 0.5)
+TURN3 = workloads.ShapeSpec("turn3", 512, 384, 4004, 1, 6, 2, 1200, 0.125, 0.3)
+TURNP = workloads.ShapeSpec("turnp", 512, 1152, 4096, 1, 18, 2, 1200, 0.125, 0.3)
+
+
+@pytest.mark.parametrize("spec,kind,n", [
+    (TURN1, "plain", 700), (TURN1, "wide", 641), (TURN3, "plain", 769),
+    (TURN3, "corrections", 650), (TURNP, "plain", 600)],
+    ids=lambda v: getattr(v, "name", str(v)))
+def test_tiles_in_turn(monkeypatch, spec, kind, n):
+    _compare(monkeypatch, spec, kind, n, 8)
+
+
 def test_oracle_replay(monkeypatch):
     """Hidden pairs and K/V rows of a prompt over three tiles against the
     oracle's task by task replay."""
