@@ -328,30 +328,52 @@ __global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 1) void pf_gemm_kernel(PfGe
         // adds the others'
         const size_t tile = (size_t)ni * mtiles + j % mtiles;
         int64_t* base = a.part + tile * parts * (size_t)(NTH * 32) + tid;
-        int64_t t[32];
-#pragma unroll
-        for (int i = 0; i < 32; i++) {
+        auto sum = [&](int i) {
             const v16i* c = acc[i >> 4];
-            t[i] = ((((int64_t)c[0][i & 15] << 8) + c[1][i & 15]) << 8) + c[2][i & 15];
-            st_coherent(base + ((size_t)part * 32 + i) * NTH, t[i]);
-        }
+            return ((((int64_t)c[0][i & 15] << 8) + c[1][i & 15]) << 8) + c[2][i & 15];
+        };
+#pragma unroll
+        for (int i = 0; i < 32; i++) st_coherent(base + ((size_t)part * 32 + i) * NTH, sum(i));
         if (!arrive_last(&a.count[tile], parts, &last)) continue;
+        // C sums of U parts requested together.  Left to itself the compiler
+        // waits for each load before the next where a thread's registers are
+        // short, two and four wavefronts: 8 us a part (down of 32 rows in
+        // eight parts 79 us, 33 so); with eight it requests all 32 by itself.
+        constexpr int C = WM == 4 ? 32 : 8;
+        constexpr uint32_t U = WM == 4 ? 1 : 4;
+#pragma unroll
+        for (int i0 = 0; i0 < 32; i0 += C) {
+            int64_t t[C];
+#pragma unroll
+            for (int i = 0; i < C; i++) t[i] = sum(i0 + i);
 #pragma unroll 1
-        for (uint32_t q = 1; q < parts; q++) {
-            const int64_t* o = base + (size_t)((part + q) % parts) * 32 * NTH;
+            for (uint32_t q0 = 1; q0 < parts; q0 += U) {
+                int64_t o[U][C];
 #pragma unroll
-            for (int i = 0; i < 32; i++) t[i] += ld_coherent(o + (size_t)i * NTH);
-        }
+                for (uint32_t u = 0; u < U; u++) {
+                    uint32_t q = part + (U == 1 ? q0 : min(q0 + u, parts - 1));
+                    q -= q >= parts ? parts : 0;
 #pragma unroll
-        for (int i = 0; i < 32; i++) {
-            // back as 256 x + bd, x far outside the narrowing's range where
-            // it does not fit
-            constexpr int64_t lim = WIDE ? INT32_MAX : 1 << 29;
-            const int64_t h = t[i] >> 8;
-            v16i* c = acc[i >> 4];
-            c[0][i & 15] = 0;
-            c[1][i & 15] = (int32_t)(h < -lim ? -lim : (h > lim ? lim : h));
-            c[2][i & 15] = (int32_t)(t[i] & 255);
+                    for (int i = 0; i < C; i++)
+                        o[u][i] = ld_coherent(base + ((size_t)q * 32 + i0 + i) * NTH);
+                }
+                if (WM < 4) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (uint32_t u = 0; u < U; u++)
+#pragma unroll
+                    for (int i = 0; i < C; i++) t[i] += U == 1 || q0 + u < parts ? o[u][i] : 0;
+            }
+#pragma unroll
+            for (int i = 0; i < C; i++) {
+                // back as 256 x + bd, x far outside the narrowing's range
+                // where it does not fit
+                constexpr int64_t lim = WIDE ? INT32_MAX : 1 << 29;
+                const int64_t h = t[i] >> 8;
+                v16i* c = acc[(i0 + i) >> 4];
+                c[0][(i0 + i) & 15] = 0;
+                c[1][(i0 + i) & 15] = (int32_t)(h < -lim ? -lim : (h > lim ? lim : h));
+                c[2][(i0 + i) & 15] = (int32_t)(t[i] & 255);
+            }
         }
     }
     // ---- epilogue: lane's element 4 g + t of piece nt is output 8 g + 4
@@ -1088,8 +1110,10 @@ hipError_t pf_gemm_w(const PfGemmArgs& a, uint32_t ntiles, uint32_t wm, hipStrea
 // while the tiles alone leave half of the 256 compute units idle: the parts'
 // exchange takes ~15 us on a full chip, a 128-input step ~1.5 us, so at least
 // 32 steps stay with a part there (down, 1,024 rows, 86 steps: 137 us whole,
-// 85 in two parts; Q|K|V, 16 steps: 33 and 47) and 8 where it is nearly
-// empty (16 rows, down: 122 us whole, 31 in eight parts; O: 28 and 22).
+// 85 in two parts; Q|K|V, 16 steps: 33 and 47).  Where it is nearly empty, 8
+// steps (128 rows, Q|K|V in 8 and in 4 steps a part: 26 us both) or, with the
+// smaller exchange of at most 64 rows, 4 (32 rows, O in two and four parts:
+// 25 and 21 us, Q|K|V 24 and 20; of 2 steps 22).
 PfShape pf_gemm_shape(uint32_t m, uint32_t n, uint32_t steps, int epi) {
     const uint32_t ntiles = epi == EPI_SILU ? (n + 127) / 128 * 2 : (n + 127) / 128;
     PfShape s;
@@ -1097,7 +1121,7 @@ PfShape pf_gemm_shape(uint32_t m, uint32_t n, uint32_t steps, int epi) {
     s.tiles = ntiles * ((m + 32 * s.wm - 1) / (32 * s.wm));
     s.parts = 1;
     while (s.parts < 8 && 2 * s.tiles * s.parts <= 256 &&
-           steps / (2 * s.parts) >= (s.tiles * s.parts >= 128 ? 32u : 8u))
+           steps / (2 * s.parts) >= (s.tiles * s.parts >= 128 ? 32u : s.wm == 4 ? 8u : 4u))
         s.parts *= 2;
     return s;
 }

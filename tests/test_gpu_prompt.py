@@ -138,6 +138,21 @@ def test_tiles_in_turn(monkeypatch, spec, kind, n):
     _compare(monkeypatch, spec, kind, n, 8)
 
 
+# K in two, four and eight parts for up to 64 rows, of unequal lengths: 40, 21 and 11
+# steps of down, 9 of Q|K|V and O.
+SPLIT40 = workloads.ShapeSpec("split40", 512, 256, 5100, 1, 4, 2, 1200, 0.25, 0.5)
+SPLIT21 = workloads.ShapeSpec("split21", 512, 1152, 2600, 1, 18, 2, 1200, 0.125, 0.3)
+SPLIT11 = workloads.ShapeSpec("split11", 512, 128, 1300, 1, 4, 2, 1200, 0.25, 0.5)
+
+
+@pytest.mark.parametrize("kind", ["plain", "wide", "corrections"])
+@pytest.mark.parametrize("spec,n", [(SPLIT40, 32), (SPLIT40, 51), (SPLIT21, 25),
+                                    (SPLIT21, 64), (SPLIT11, 30)],
+                         ids=lambda v: getattr(v, "name", str(v)))
+def test_split_products(monkeypatch, spec, n, kind):
+    _compare(monkeypatch, spec, kind, n, 6)
+
+
 def test_oracle_replay(monkeypatch):
     """Hidden pairs and K/V rows of a prompt over three tiles against the
     oracle's task by task replay."""
