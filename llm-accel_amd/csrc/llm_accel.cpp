@@ -2408,9 +2408,16 @@ int run_stack(llm_ctx_t* c, const int16_t* rows_host, uint32_t rows, uint32_t po
 }
 
 // Rows of a prompt that go through a layer at once (its workspace is bounded
-// by them), and the blocks from which that is the faster way: one layer of
-// config B takes 51 us per 8-row block and ~145 us for 16 to 32 rows at once.
-constexpr uint32_t kPfMaxRows = 2048, kPfMinBlocks = 4;
+// by them), and the blocks from which that is the faster way: one layer takes
+// ~128 us for up to 32 rows at once on config B (91 at hidden 896, 70 at 480,
+// 57 at 256), and in blocks of 8 or 5 rows 180 / 115 / 93 / 91 us for four of
+// them, 136 / 88 / 71 / 69 for three; in one-row blocks 139 / 81 / 70 / 64 for
+// four.  With matrices held in 16 bits 183 / 124 / 93 / 75 against 195 / 110 /
+// 86 / 83 for four blocks: six.
+constexpr uint32_t kPfMaxRows = 2048;
+constexpr uint32_t pf_min_blocks(uint32_t block, bool wide) {
+    return (block > 1 ? 4 : 5) + (wide ? 2 : 0);
+}
 // Split-K scratch of its products: at most 256 workgroup parts of 128 x 128
 // 64-bit sums, and their arrival counters.
 constexpr size_t kPfPartBytes = (size_t)256 * 128 * 128 * 8;
@@ -2419,17 +2426,20 @@ constexpr uint32_t kPfMaxTiles = 256;
 // Whether every matrix of layers [0, layer_count) has a layout that the
 // layer-major prompt path reads.
 bool prompt_path_ok(llm_ctx* c, uint32_t n_prompt, uint32_t block, uint32_t layer_count) {
-    if (!c->prompt_path || c->const_gain <= 0 || c->log_fn || cdiv(n_prompt, block) < kPfMinBlocks)
+    const uint32_t blocks = cdiv(n_prompt, block);
+    if (!c->prompt_path || c->const_gain <= 0 || c->log_fn || blocks < pf_min_blocks(block, false))
         return false;
+    bool wide = false;
     for (uint32_t l = 0; l < layer_count; l++) {
         for (int m = 0; m < M_COUNT; m++) {
             const Matrix& mt = c->mat(l, m);
             if (mt.steps > llm::kP12MaxSteps || (!mt.p12_ok && !mt.mf)) return false;
+            wide |= !mt.p12_ok;
         }
         const Matrix &g = c->mat(l, M_GATE), &u = c->mat(l, M_UP);
         if (!(g.p12_ok && u.p12_ok) && !(g.mf && u.mf)) return false;
     }
-    return true;
+    return blocks >= pf_min_blocks(block, wide);
 }
 
 int prompt_buffers(llm_ctx* c, uint32_t rows) {

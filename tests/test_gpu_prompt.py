@@ -100,7 +100,7 @@ def _compare(monkeypatch, spec, kind, n, block, gen=1):
     assert got[4] == want[4]
 
 
-@pytest.mark.parametrize("n,block", [(4, 1), (31, 8), (33, 5), (64, 8), (65, 8), (127, 3),
+@pytest.mark.parametrize("n,block", [(4, 1), (5, 1), (31, 8), (33, 5), (64, 8), (65, 8), (127, 3),
                                      (129, 8), (200, 7)])
 def test_row_counts(monkeypatch, n, block):
     _compare(monkeypatch, D64, "plain", n, block)
@@ -150,7 +150,7 @@ SPLIT11 = workloads.ShapeSpec("split11", 512, 128, 1300, 1, 4, 2, 1200, 0.25, 0.
                                     (SPLIT21, 64), (SPLIT11, 30)],
                          ids=lambda v: getattr(v, "name", str(v)))
 def test_split_products(monkeypatch, spec, n, kind):
-    _compare(monkeypatch, spec, kind, n, 6)
+    _compare(monkeypatch, spec, kind, n, 4)
 
 
 def test_oracle_replay(monkeypatch):
