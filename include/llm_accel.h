@@ -21,8 +21,15 @@
  *   - KV cache preload / inspection (host/host_qwen_8x64.cpp:1729-1843)
  *     -> llm_kv_write(), llm_kv_read().
  *
- * Threading: one host thread per context; every call is synchronous with
- * respect to the caller (work runs on the context's own HIP stream).
+ * Threading: one host thread per context.  Work runs on the context's own
+ * HIP stream: llm_task() and llm_op() enqueue it; every call that returns
+ * results to host memory, and llm_sync(), waits for what was enqueued
+ * before.  Host memory that a call reads is the caller's again when the
+ * call returns, and rows copied into a pair or port are in place for every
+ * later call of the context and, from the moment llm_pair_device_ptr(),
+ * llm_port() or llm_stream() has returned, for every other reader: those
+ * three wait for copies under way, and once the address (of a pair, of the
+ * ports) or the stream is out, copies are complete on return.
  * Return values: >= 0 is a reference status code (llm_task) or 0; < 0 is an
  * error of this library (LLM_E_*), with a message in llm_last_error().
  */
@@ -237,8 +244,10 @@ int llm_op(llm_ctx_t* ctx, uint32_t op, uint32_t layer, uint32_t token_count,
  * the reference host's six data buffers data_words_ (two per port name,
  * host/host_qwen_8x64.cpp:3060, packed by :2062-2123). */
 int llm_port(llm_ctx_t* ctx, uint32_t port, void** dev, size_t* elems);
-/* Synchronous host copies into / out of a port buffer (the migrations
- * around launch(), host/host_qwen_8x64.cpp:2500-2757). */
+/* Host copies into / out of a port buffer (the migrations around launch(),
+ * host/host_qwen_8x64.cpp:2500-2757).  A write is ordered before everything
+ * enqueued later and complete on return once llm_port() or llm_stream() was
+ * called; a read waits for everything enqueued before it. */
 int llm_port_write(llm_ctx_t* ctx, uint32_t port, const int16_t* host, size_t elems);
 int llm_port_read(llm_ctx_t* ctx, uint32_t port, int16_t* host, size_t elems);
 
@@ -252,7 +261,8 @@ int llm_kv_write(llm_ctx_t* ctx, uint32_t layer, uint32_t kv_head,
 /* Zero the whole KV cache (accelerator_t constructor, host:1073-1074). */
 int llm_kv_clear(llm_ctx_t* ctx);
 
-/* Device pointer of a pair's [8][hidden] rows (for zero-copy callers). */
+/* Device pointer of a pair's [8][hidden] rows (for zero-copy callers);
+ * waits for copies into pairs and ports under way. */
 void* llm_pair_device_ptr(llm_ctx_t* ctx, uint32_t pair);
 /* The context's HIP stream (hipStream_t) and a full synchronisation. */
 void* llm_stream(llm_ctx_t* ctx);

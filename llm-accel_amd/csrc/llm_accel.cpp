@@ -277,7 +277,9 @@ struct llm_ctx {
     // to its number once its values are visible, and a device word for its
     // workgroups' arrivals.  `busy`: what has been enqueued since a transfer
     // or synchronisation was last seen to complete (not relied on once the
-    // stream was handed out).
+    // stream was handed out; from then on no copy into a pair or port is left
+    // under way either, so that no other call has to wait on a stream that
+    // the caller may be capturing).
     int16_t *io_in = nullptr, *io_out = nullptr;
     size_t io_elems = 0;
     uint32_t* io_flag = nullptr;
@@ -286,6 +288,7 @@ struct llm_ctx {
     enum Busy { QUIET, COPIES_IN, WORK };
     Busy busy = WORK;
     bool stream_out = false;
+    bool copies_open = false;  // a copy into a pair or port may be under way
     size_t io_used = 0;   // of io_in, by copies not known to be complete
     uint64_t n_h2d_rows = 0;   // hidden-row uploads (calls)
     uint64_t n_d2h_rows = 0;   // hidden-row downloads (calls)
@@ -414,6 +417,7 @@ int io_wait(llm_ctx* c, uint32_t seq) {
     for (uint32_t i = 0; i < 200000; i++) {
         if (__atomic_load_n(c->io_flag, __ATOMIC_ACQUIRE) == seq) {
             c->busy = llm_ctx::QUIET;
+            c->copies_open = false;
             return 0;
         }
         __builtin_ia32_pause();
@@ -422,11 +426,23 @@ int io_wait(llm_ctx* c, uint32_t seq) {
     if (__atomic_load_n(c->io_flag, __ATOMIC_ACQUIRE) != seq)
         return fail(LLM_E_HIP, "a transfer to the host did not complete");
     c->busy = llm_ctx::QUIET;
+    c->copies_open = false;
+    return 0;
+}
+
+// Every copy into a pair or port has completed: before the caller receives
+// an address or the stream, through which it can reach the values without a
+// call that waits for them.  Leaves `busy` and a wait that gave up to the
+// next call that reports it.
+int finish_copies(llm_ctx* c) {
+    if (!c->copies_open) return 0;
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    c->copies_open = false;
     return 0;
 }
 
 // Rows of `cols` values from host memory into device rows: staged, the copy
-// enqueued and, unless `wait`, not waited for.
+// enqueued and, unless `wait` or the stream was handed out, not waited for.
 int rows_in(llm_ctx* c, const int16_t* host, int16_t* dev, uint32_t ld_dev, uint32_t cols,
             uint32_t rows, bool wait) {
     bool late = false;
@@ -445,7 +461,9 @@ int rows_in(llm_ctx* c, const int16_t* host, int16_t* dev, uint32_t ld_dev, uint
         HIP_TRY(llm::launch_io_rows(from, cols, dev, ld_dev, cols, rows, nullptr, nullptr, 0,
                                     c->stream));
         c->busy = llm_ctx::COPIES_IN;
-        if (wait) HIP_TRY(hipStreamSynchronize(c->stream));
+        c->copies_open = true;
+        if (wait || c->stream_out)
+            if (int rc = finish_copies(c)) return rc;
     }
     return late ? late_error() : 0;
 }
@@ -1870,8 +1888,9 @@ int llm_port(llm_ctx_t* c, uint32_t port, void** dev, size_t* elems) {
     HIP_TRY(hipSetDevice(c->device));
     if (int rc = ensure_ports(c)) return rc;
     if (dev) {
+        if (int rc = finish_copies(c)) return rc;
         *dev = c->ports[port];
-        c->port_out = true;  // port writes stay complete on return
+        c->port_out = true;  // from here on port writes are complete on return
     }
     if (elems) *elems = c->port_n;
     return 0;
@@ -2082,6 +2101,7 @@ int llm_kv_clear(llm_ctx_t* c) {
 void* llm_pair_device_ptr(llm_ctx_t* c, uint32_t pair) {
     if (!c || pair >= c->pairs.size()) return nullptr;
     if (hipSetDevice(c->device) != hipSuccess) return nullptr;
+    if (finish_copies(c) != 0) return nullptr;
     invalidate_pair(c, (int)pair);  // the caller may write through it
     c->exported[pair] = 1;          // and keeps using this address
     return c->pairs[pair];
@@ -2090,6 +2110,7 @@ void* llm_pair_device_ptr(llm_ctx_t* c, uint32_t pair) {
 void* llm_stream(llm_ctx_t* c) {
     if (!c) return nullptr;
     if (hipSetDevice(c->device) != hipSuccess) return nullptr;
+    if (finish_copies(c) != 0) return nullptr;
     c->stream_out = true;  // the caller may enqueue on it
     return (void*)c->stream;
 }

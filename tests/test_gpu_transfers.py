@@ -1,7 +1,9 @@
 """Rows and ports between host and device (copy kernels over pinned staging): sizes that
 end within a 16-byte piece or a workgroup, uploads that follow one another, fill the
-staging or overtake running tasks, and projections that read their rows from the port or
-from elsewhere."""
+staging or overtake running tasks, projections that read their rows from the port or
+from elsewhere, and copies that are complete once an address is in the caller's hands."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -79,3 +81,61 @@ def test_projection_rows_from_anywhere(ctx, rows):
         assert st.code == 0
         got = acc.port_read(L.PORT_OUT if dst == p_out else L.PORT_IN, want.size)
         assert np.array_equal(got.reshape(want.shape), want), (port, shift, dst == p_in)
+
+
+class _Memory:
+    """Copies through the HIP runtime that the library links, on the null stream: the
+    context's stream does not wait for it, nor it for the context's."""
+
+    def __init__(self):
+        self.rt = ctypes.CDLL("libamdhip64.so.7")
+
+    def read(self, dev, n):
+        a = np.zeros(n, np.int16)
+        assert self.rt.hipMemcpy(a.ctypes.data_as(ctypes.c_void_p), ctypes.c_void_p(dev),
+                                 ctypes.c_size_t(2 * n), 2) == 0
+        return a
+
+    def write(self, dev, a):
+        a = np.ascontiguousarray(a)
+        assert self.rt.hipMemcpy(ctypes.c_void_p(dev), a.ctypes.data_as(ctypes.c_void_p),
+                                 ctypes.c_size_t(a.nbytes), 1) == 0
+
+
+@pytest.mark.parametrize("stream_out", [False, True])
+def test_copies_are_complete_when_an_address_is_handed_out(stream_out):
+    """Uploads and port writes under way when the address is asked for the first time:
+    what another stream reads through it is the new rows, and what it writes through it
+    stays.  Then the same with the address in hand, and with the stream in hand."""
+    import llm_accel as L
+    hidden, inter, pairs = 2048, 11008, 10
+    rng = np.random.default_rng(11 + stream_out)
+    mem = _Memory()
+    with L.Accelerator(L.Shape(64, hidden, inter, 1, 16, 2, 64, 1e6), num_pairs=pairs) as acc:
+        if stream_out:
+            assert L.lib().llm_stream(acc._ctx)
+        for p in range(1, pairs):
+            for again in range(2):  # the first time the address leaves, then with it known
+                acc.sync()
+                rows = [_ints(rng, (8, hidden)) for _ in range(4)]
+                for i in range(8):  # copies that the last one stands behind
+                    acc.upload(0, rows[i % 3])
+                acc.upload(p, rows[3])
+                ptr = L.lib().llm_pair_device_ptr(acc._ctx, p)
+                assert np.array_equal(mem.read(ptr, rows[3].size), rows[3].reshape(-1)), (p, again)
+                acc.upload(p, rows[0])
+                if not again:
+                    ptr = L.lib().llm_pair_device_ptr(acc._ctx, p)
+                mem.write(ptr, rows[1])
+                assert np.array_equal(acc.download(p, 8), rows[1]), (p, again)
+        n = 8 * inter
+        for port in (L.PORT_IN, L.PORT_AUX, L.PORT_OUT):
+            x, y = _ints(rng, n), _ints(rng, n)
+            acc.sync()
+            acc.port_write(port, y)
+            acc.port_write(port, x)
+            dev, _ = acc.port(port)
+            assert np.array_equal(mem.read(dev, n), x), port
+            acc.port_write(port, y)
+            mem.write(dev, x)
+            assert np.array_equal(acc.port_read(port, n), x), port
