@@ -516,7 +516,10 @@ int dev_alloc(llm_ctx* c, void** p, size_t bytes) {
         return fail(LLM_E_NOMEM, "hipMalloc(" + std::to_string(bytes) +
                                      "): " + hipGetErrorString(e));
     c->allocations.push_back(*p);
+    // the fill runs behind the call, on the null stream, which the context's
+    // non-blocking stream does not wait for
     e = hipMemset(*p, 0, bytes);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return fail(LLM_E_HIP, hipGetErrorString(e));
     return 0;
 }
@@ -1418,8 +1421,6 @@ int llm_ctx_create(const llm_shape_t* shape, int device, uint32_t num_pairs,
         if ((rc = dev_alloc(c, (void**)&c->mf_part, words * 4)) ||
             (rc = dev_alloc(c, (void**)&c->mf_count, chunks * 4)))
             return cleanup(rc);
-        if (hipMemset(c->mf_count, 0, chunks * 4) != hipSuccess)
-            return cleanup(fail(LLM_E_HIP, "hipMemset failed"));
         for (auto& mt : c->mats) {
             mt.ctx_part = c->mf_part;
             mt.ctx_count = c->mf_count;

@@ -153,6 +153,32 @@ def test_split_products(monkeypatch, spec, n, kind):
     _compare(monkeypatch, spec, kind, n, 4)
 
 
+def test_prompts_that_outgrow_the_workspace(monkeypatch):
+    """One context, prompts of growing and falling length: each is the first work on a
+    workspace that has just been allocated, or runs in a larger one."""
+    import llm_accel
+    spec = D128
+    model = Model(spec, "plain")
+    rng = np.random.default_rng(23)
+    prompts = [[int(t) for t in rng.integers(0, spec.vocab, size=n)] for n in (40, 300, 1100, 90)]
+    got = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("LLM_ACCEL_PROMPT", mode)
+        with llm_accel.Accelerator(accel_shape(spec)) as a:
+            a.load_model(model)
+            a.load_lm_head(model.emb)
+            for prompt in prompts:
+                toks, _ = a.generate(model.emb, prompt, 8, spec.layers, 2)
+                kv = [a.kv_read(layer, h, 0, len(prompt)) for layer in range(spec.layers)
+                      for h in range(spec.kv_heads)]
+                got.setdefault(mode, []).append((toks, a.download(0, 8), a.download(1, 8), kv))
+    for n, (want, have) in zip(map(len, prompts), zip(got["0"], got["1"])):
+        assert have[0] == want[0], n
+        assert np.array_equal(have[1], want[1]) and np.array_equal(have[2], want[2]), n
+        for i, ((k0, v0), (k1, v1)) in enumerate(zip(want[3], have[3])):
+            assert np.array_equal(k0, k1) and np.array_equal(v0, v1), (n, i)
+
+
 def test_oracle_replay(monkeypatch):
     """Hidden pairs and K/V rows of a prompt over three tiles against the
     oracle's task by task replay."""

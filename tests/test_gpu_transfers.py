@@ -139,3 +139,18 @@ def test_copies_are_complete_when_an_address_is_handed_out(stream_out):
             acc.port_write(port, y)
             mem.write(dev, x)
             assert np.array_equal(acc.port_read(port, n), x), port
+
+
+def test_first_writes_of_new_buffers():
+    """Rows and ports written as the first thing that happens to their memory, which the
+    allocation's fill with zeros must not overtake: large contexts, whose fills take long."""
+    import llm_accel as L
+    rng = np.random.default_rng(17)
+    for _ in range(4):
+        rows, port = _ints(rng, (8, 2048)), _ints(rng, 8 * 11008)
+        with L.Accelerator(L.Shape(64, 2048, 11008, 1, 16, 2, 16384, 1e6), num_pairs=64) as acc:
+            acc.upload(63, rows)
+            acc.port_write(L.PORT_OUT, port)
+            acc.sync()
+            assert np.array_equal(acc.download(63, 8), rows)
+            assert np.array_equal(acc.port_read(L.PORT_OUT, port.size), port)
