@@ -1197,13 +1197,20 @@ static hipError_t launch_lm_rt(const int16_t* w, uint32_t steps, uint32_t n,
                                const int16_t* x, uint32_t ldx, uint32_t rows, int L,
                                unsigned long long* keys, hipStream_t st) {
     const uint32_t nblocks = (n + 3) / 4;
-    // Every workgroup ends with one atomicMax on the same line: 384 of them,
-    // three per two compute units, not one per four blocks (16,384 rows of
-    // 2,048 / 896: call 29.3 / 23.1 us with up to 2,048 workgroups, 21.9 /
-    // 16.6 with 384, 24.0 / 17.9 with 512; 151,936 rows of 2,048 115 -> 109).
-    uint32_t grid = (nblocks + 3) / 4;
-    if (grid > 384) grid = 384;
-    if (RT <= 2 && steps <= kLmStageSteps) {
+    // Every workgroup ends with one atomicMax per row on the same line, and
+    // every wavefront adds to the loads in flight.  One staged row streams the
+    // table from 384 workgroups, three per two compute units (call us with at
+    // most 384 / 2,048: 16,384 x 896 16.7 / 22.7, 32,000 x 2,048 29.3 / 41.4,
+    // 151,936 x 2,048 108 / 112).  Two staged rows need more wavefronts once
+    // the table is large (151,936 x 2,048 225 / 119), fewer where it is small
+    // (16,384 x 896 18.3 / 23.6): four blocks a wavefront.  Rows read from
+    // memory wait for them in the loop and need them all (32,000 x 5,120, 1,
+    // 2, 3 and 8 rows of full range: 140, 205, 340, 541 / 73, 89, 117, 254).
+    const bool staged = RT <= 2 && steps <= kLmStageSteps;
+    const uint32_t cap =
+        !staged ? 2048 : (RT == 1 ? 384 : std::min(std::max(nblocks / 16, 384u), 2048u));
+    const uint32_t grid = std::min((nblocks + 3) / 4, cap);
+    if (staged) {
         constexpr bool XS = RT <= 2;
         switch (L) {
         case 0: lm_argmax_kernel<RT, 0, XS><<<grid, 256, 0, st>>>(w, steps, n, x, ldx, rows, keys); break;
