@@ -402,7 +402,11 @@ int llm_set_log(llm_ctx_t* ctx, llm_log_fn fn, void* user);
  * A prompt of several blocks runs layer by layer over many rows at once
  * (no line sink set, hidden >= 128): every row's values, the K/V cache, the
  * hidden pairs and the counts are those of the block by block loop, and
- * prompt_forward_ms is the time of the whole.
+ * prompt_forward_ms is the time of the whole.  The first such prompt
+ * allocates device memory that the context keeps, and a longer one more:
+ * about 20 hidden + 2 intermediate bytes per prompt row (2,048 rows at
+ * most), four bytes per element of one layer's K rows, and 34 MB.  Where
+ * that cannot be had fewer rows run at a time, or the prompt in blocks.
  * A one-launch kernel whose bounded wait between workgroups gives up
  * (e.g. a device shared with other work) does not fail the request: the
  * forwards since the previous synchronisation run again on launches

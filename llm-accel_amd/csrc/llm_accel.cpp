@@ -259,7 +259,9 @@ struct llm_ctx {
     // Layer-major prompt path (prefill.h) of llm_generate: its buffers, one
     // allocation sized for `rows` rows (a multiple of kPfRowPad), made by the
     // first prompt that takes it and replaced by a larger one when a longer
-    // prompt comes; LLM_ACCEL_PROMPT=0 keeps the prompt in blocks
+    // prompt comes.  Where the device has no room for it, or it would pass
+    // LLM_ACCEL_PROMPT_BYTES, fewer rows run at a time, or the prompt in
+    // blocks; LLM_ACCEL_PROMPT=0 keeps every prompt in blocks
     struct Prompt {
         uint32_t rows = 0;
         uint8_t* base = nullptr;
@@ -272,6 +274,7 @@ struct llm_ctx {
         size_t part_bytes = 0;
     } pf;
     bool prompt_path = true;
+    size_t prompt_bytes = SIZE_MAX;
     // Transfers of rows and keys with the host: pinned staging (in: host to
     // device, out: device to host), the pinned word a transfer's kernel sets
     // to its number once its values are visible, and a device word for its
@@ -512,9 +515,11 @@ struct WaitFreeScope {
 
 int dev_alloc(llm_ctx* c, void** p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // not the next launch's
         return fail(LLM_E_NOMEM, "hipMalloc(" + std::to_string(bytes) +
                                      "): " + hipGetErrorString(e));
+    }
     c->allocations.push_back(*p);
     // the fill runs behind the call, on the null stream, which the context's
     // non-blocking stream does not wait for
@@ -1361,6 +1366,8 @@ int llm_ctx_create(const llm_shape_t* shape, int device, uint32_t num_pairs,
     if (const char* e = std::getenv("LLM_ACCEL_FUSED")) c->fused = std::strcmp(e, "0") != 0;
     if (const char* e = std::getenv("LLM_ACCEL_PROMPT"))
         c->prompt_path = std::strcmp(e, "0") != 0;
+    if (const char* e = std::getenv("LLM_ACCEL_PROMPT_BYTES"))
+        c->prompt_bytes = (size_t)std::strtoull(e, nullptr, 10);
     if (const char* e = std::getenv("LLM_ACCEL_GQA")) c->gqa = std::strcmp(e, "0") != 0;
     if (const char* e = std::getenv("LLM_ACCEL_TILE_FUSED"))
         c->tile_fused = std::strcmp(e, "0") != 0;
@@ -2464,69 +2471,72 @@ bool prompt_path_ok(llm_ctx* c, uint32_t n_prompt, uint32_t block, uint32_t laye
     return blocks >= pf_min_blocks(block, wide);
 }
 
-int prompt_buffers(llm_ctx* c, uint32_t rows) {
-    auto& p = c->pf;
-    const uint32_t R = round_up(rows, llm::kPfRowPad);
-    if (p.rows >= R) return 0;
-    if (p.base) {
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        if (int rc = dev_free(c, p.base)) return rc;
-        p = {};
-    }
+// Places the buffers for p.rows rows from p.base on (nowhere while that is
+// null); returns their bytes.
+size_t place_prompt_buffers(const llm_ctx* c, llm_ctx::Prompt& p) {
     size_t at = 0;
-    auto take = [&](size_t bytes) {
-        const size_t o = at;
+    auto take = [&](auto*& ptr, size_t bytes) {
+        ptr = p.base ? (std::remove_reference_t<decltype(ptr)>)(p.base + at) : nullptr;
         at += (bytes + 255) / 256 * 256;
-        return o;
     };
-    const uint32_t np = round_up(c->Nqkv, 128);
-    const size_t o_in = take((size_t)R * c->H * 2), o_ha = take((size_t)R * c->Hp * 2),
-                 o_hb = take((size_t)R * c->Hp * 2), o_qkv = take((size_t)R * np * 2),
-                 o_xn = take(llm::pf_xp_bytes(R, c->Hp)), o_xa = take(llm::pf_xp_bytes(R, c->Hp)),
-                 o_act = take(llm::pf_xp_bytes(R, c->Ip)),
-                 o_qp = take(llm::pf_qp_bytes(R, c->Hq, c->d)),
-                 o_kp = take(llm::pf_kp_bytes(c->Hkv, c->tiles, c->d)),
-                 o_vp = take(llm::pf_vp_bytes(c->Hkv, c->tiles, c->d)),
-                 o_kb = take((size_t)c->Hkv * c->tiles * 64 * 4), o_rs = take((size_t)R * 4),
-                 o_kf = take((size_t)2 * c->Hkv * c->tiles * 4),
-                 o_qf = take((size_t)c->Hq * (R / 32) * 4), o_ct = take(kPfMaxTiles * 4),
-                 o_pt = take(kPfPartBytes);
-    uint8_t* b = nullptr;
-    if (int rc = dev_alloc(c, (void**)&b, at)) return rc;
-    p.base = b;
-    p.in = (int16_t*)(b + o_in);
-    p.ha = (int16_t*)(b + o_ha);
-    p.hb = (int16_t*)(b + o_hb);
-    p.qkv = (int16_t*)(b + o_qkv);
-    p.xn = (int8_t*)(b + o_xn);
-    p.xa = (int8_t*)(b + o_xa);
-    p.act = (int8_t*)(b + o_act);
-    p.qp = (int8_t*)(b + o_qp);
-    p.kp = (int8_t*)(b + o_kp);
-    p.vp = (int8_t*)(b + o_vp);
-    p.kbias = (int32_t*)(b + o_kb);
-    p.rowsum = (int32_t*)(b + o_rs);
-    p.kvflag = (uint32_t*)(b + o_kf);
-    p.qflag = (uint32_t*)(b + o_qf);
-    p.count = (uint32_t*)(b + o_ct);
-    p.part = (int64_t*)(b + o_pt);
+    const size_t R = p.rows, np = round_up(c->Nqkv, 128);
+    take(p.in, R * c->H * 2);
+    take(p.ha, R * c->Hp * 2);
+    take(p.hb, R * c->Hp * 2);
+    take(p.qkv, R * np * 2);
+    take(p.xn, llm::pf_xp_bytes(p.rows, c->Hp));
+    take(p.xa, llm::pf_xp_bytes(p.rows, c->Hp));
+    take(p.act, llm::pf_xp_bytes(p.rows, c->Ip));
+    take(p.qp, llm::pf_qp_bytes(p.rows, c->Hq, c->d));
+    take(p.kp, llm::pf_kp_bytes(c->Hkv, c->tiles, c->d));
+    take(p.vp, llm::pf_vp_bytes(c->Hkv, c->tiles, c->d));
+    take(p.kbias, (size_t)c->Hkv * c->tiles * 64 * 4);
+    take(p.rowsum, R * 4);
+    take(p.kvflag, (size_t)2 * c->Hkv * c->tiles * 4);
+    take(p.qflag, (size_t)c->Hq * (R / 32) * 4);
+    take(p.count, kPfMaxTiles * 4);
+    take(p.part, kPfPartBytes);
     p.part_bytes = kPfPartBytes;
-    // attention outputs past the heads' width stay 0 (the attention writes
-    // whole heads only)
-    HIP_TRY(llm::launch_pf_init(p.in, R, 0, c->Hp, c->norms, c->const_gain, p.ha, p.xa, c->stream));
-    p.rows = R;
+    return at;
+}
+
+// Buffers for `rows` rows at a time or, where there is no room for them, for
+// as many (half, a quarter, ...) as there is: c->pf.rows, 0 if for none.  The
+// buffers in hand are given up only for larger ones.
+int prompt_buffers(llm_ctx* c, uint32_t rows) {
+    const uint32_t pad = llm::kPfRowPad;
+    for (uint32_t R = round_up(rows, pad); R > c->pf.rows; R = R > pad ? round_up(R / 2, pad) : 0) {
+        llm_ctx::Prompt p{};
+        p.rows = R;
+        const size_t bytes = place_prompt_buffers(c, p);
+        if (bytes > c->prompt_bytes) continue;
+        const int rc = dev_alloc(c, (void**)&p.base, bytes);
+        if (rc == LLM_E_NOMEM) continue;
+        if (rc) return rc;
+        place_prompt_buffers(c, p);
+        if (c->pf.base) {
+            HIP_TRY(hipStreamSynchronize(c->stream));
+            if (int r = dev_free(c, c->pf.base)) return r;
+        }
+        c->pf = p;
+        // attention outputs past the heads' width stay 0 (the attention
+        // writes whole heads only)
+        HIP_TRY(llm::launch_pf_init(p.in, R, 0, c->Hp, c->norms, c->const_gain, p.ha, p.xa,
+                                    c->stream));
+        break;
+    }
     return 0;
 }
 
 // Prompt rows [0, n) (pinned host memory) through layers [0, layer_count),
-// layer by layer over up to kPfMaxRows rows at a time: K/V rows, hidden
-// pairs and final norm as the blocks of `block` rows leave them.
+// layer by layer over as many rows at a time as the buffers hold, at most
+// kPfMaxRows: K/V rows, hidden pairs and final norm as the blocks of `block`
+// rows leave them.
 int run_prompt_layers(llm_ctx* c, const int16_t* rows_host, uint32_t n, uint32_t block,
                       uint32_t layer_count) {
     hipStream_t st = c->stream;
-    const uint32_t chunk = std::min(n, kPfMaxRows / block * block);
-    if (int rc = prompt_buffers(c, chunk)) return rc;
     auto& p = c->pf;
+    const uint32_t chunk = std::min(n, std::min(p.rows, kPfMaxRows) / block * block);
     auto gemm = [&](const int8_t* x, uint32_t m, const Matrix& w, const Matrix* w2, int epi,
                     const int16_t* res, int16_t* out, int8_t* xp, const int16_t* gamma) -> int {
         llm::PfGemmArgs a{};
@@ -2769,7 +2779,11 @@ int llm_generate(llm_ctx_t* c, const int16_t* embedding, uint32_t vocab,
     auto run_prompt = [&](bool count) -> int {
         uint32_t uncounted = 0;
         HIP_TRY(hipEventRecord(ev_p0, c->stream));
-        if (prompt_path_ok(c, n_prompt, block_size, layer_count)) {
+        const bool layers = prompt_path_ok(c, n_prompt, block_size, layer_count);
+        if (layers)
+            if (int r = prompt_buffers(c, std::min(n_prompt, kPfMaxRows / block_size * block_size)))
+                return r;
+        if (layers && c->pf.rows) {
             if (int r = run_prompt_layers(c, c->stage, n_prompt, block_size, layer_count)) return r;
             const uint32_t blocks = (uint32_t)cdiv(n_prompt, block_size);
             if (count) {

@@ -179,6 +179,64 @@ def test_prompts_that_outgrow_the_workspace(monkeypatch):
             assert np.array_equal(k0, k1) and np.array_equal(v0, v1), (n, i)
 
 
+def _bounded(monkeypatch, spec, model, prompts, block, limit):
+    """One context whose prompt buffers may take `limit` bytes (None: any): per prompt
+    its token, pairs, K/V rows and how often a layer ran over rows of it (0: in blocks)."""
+    import llm_accel
+    monkeypatch.setenv("LLM_ACCEL_PROMPT", "1")
+    monkeypatch.delenv("LLM_ACCEL_PROMPT_BYTES", raising=False)
+    if limit is not None:
+        monkeypatch.setenv("LLM_ACCEL_PROMPT_BYTES", str(int(limit)))
+    out = []
+    with llm_accel.Accelerator(accel_shape(spec)) as a:
+        a.load_model(model)
+        a.load_lm_head(model.emb)
+        for prompt in prompts:
+            a.kernel_timing(True)
+            toks, _ = a.generate(model.emb, prompt, block, spec.layers, 1)
+            times = a.kernel_stats()["rope"][0]
+            assert times % spec.layers == 0
+            kv = [a.kv_read(layer, h, 0, len(prompt)) for layer in range(spec.layers)
+                  for h in range(spec.kv_heads)]
+            out.append((toks, a.download(0, 8), a.download(1, 8), kv, times // spec.layers))
+    return out
+
+
+@pytest.mark.parametrize("block", [8, 7])
+def test_no_room_for_the_workspace(monkeypatch, block):
+    """A workspace that cannot be had in full: fewer rows at a time, at last the prompt
+    in blocks; the same results, and no error."""
+    spec, model = D64, Model(D64, "plain")
+    prompt = [int(t) for t in np.random.default_rng(31).integers(0, spec.vocab, size=1100)]
+    want, = _bounded(monkeypatch, spec, model, [prompt], block, None)
+    assert want[4] == 1
+    seen = []
+    for limit in (41e6, 37e6, 35.9e6, 35.2e6, 30e6, 0):
+        got, = _bounded(monkeypatch, spec, model, [prompt], block, limit)
+        _say(f"case blocks of {block}, workspace of {limit / 1e6:.1f} MB: {got[4]} parts")
+        assert got[0] == want[0]
+        assert np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2])
+        for i, ((k0, v0), (k1, v1)) in enumerate(zip(want[3], got[3])):
+            assert np.array_equal(k0, k1) and np.array_equal(v0, v1), i
+        seen.append(got[4])
+    assert seen[0] > 1 and seen[:4] == sorted(set(seen[:4])) and seen[4:] == [0, 0], seen
+
+
+def test_workspace_that_cannot_grow(monkeypatch):
+    """A longer prompt than the buffers in hand, and no room for larger ones: it runs in
+    those, and so does the next."""
+    spec, model = D64, Model(D64, "plain")
+    rng = np.random.default_rng(37)
+    prompts = [[int(t) for t in rng.integers(0, spec.vocab, size=n)] for n in (100, 500, 90)]
+    want = _bounded(monkeypatch, spec, model, prompts, 8, None)
+    got = _bounded(monkeypatch, spec, model, prompts, 8, 35.2e6)
+    assert [w[4] for w in want] == [1, 1, 1] and [g[4] for g in got] == [1, 4, 1]
+    for w, g in zip(want, got):
+        assert g[0] == w[0] and np.array_equal(g[1], w[1]) and np.array_equal(g[2], w[2])
+        for (k0, v0), (k1, v1) in zip(w[3], g[3]):
+            assert np.array_equal(k0, k1) and np.array_equal(v0, v1)
+
+
 def test_oracle_replay(monkeypatch):
     """Hidden pairs and K/V rows of a prompt over three tiles against the
     oracle's task by task replay."""
