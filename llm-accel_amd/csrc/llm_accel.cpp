@@ -2441,11 +2441,16 @@ int run_stack(llm_ctx_t* c, const int16_t* rows_host, uint32_t rows, uint32_t po
 // ~128 us for up to 32 rows at once on config B (91 at hidden 896, 70 at 480,
 // 57 at 256), and in blocks of 8 or 5 rows 180 / 115 / 93 / 91 us for four of
 // them, 136 / 88 / 71 / 69 for three; in one-row blocks 139 / 81 / 70 / 64 for
-// four.  With matrices held in 16 bits 183 / 124 / 93 / 75 against 195 / 110 /
-// 86 / 83 for four blocks: six.
+// four.  Every launch whose matrices have corrections adds ~15 us to a layer
+// (all four, hidden 2,048 / 896 / 512 / 256: 163 / 130 / 104 / 86 against 163
+// / 113 / 92 / 87 for four blocks of 8, 210 / 143 / 117 / 112 for five, and
+// 206 / 125 / 103 / 92 for five of two; one of the four, hidden 896: 105
+// against 112 for four): from two launches a layer on one block more.  With
+// matrices held in 16 bits 183 / 124 / 93 / 75 against 195 / 110 / 86 / 83
+// for four blocks: six.
 constexpr uint32_t kPfMaxRows = 2048;
-constexpr uint32_t pf_min_blocks(uint32_t block, bool wide) {
-    return (block > 1 ? 4 : 5) + (wide ? 2 : 0);
+constexpr uint32_t pf_min_blocks(uint32_t block, bool corr, bool wide) {
+    return (block > 1 ? 4 : 5) + (wide ? 2 : (corr ? 1 : 0));
 }
 // Split-K scratch of its products: at most 256 workgroup parts of 128 x 128
 // 64-bit sums, and their arrival counters.
@@ -2456,9 +2461,10 @@ constexpr uint32_t kPfMaxTiles = 256;
 // layer-major prompt path reads.
 bool prompt_path_ok(llm_ctx* c, uint32_t n_prompt, uint32_t block, uint32_t layer_count) {
     const uint32_t blocks = cdiv(n_prompt, block);
-    if (!c->prompt_path || c->const_gain <= 0 || c->log_fn || blocks < pf_min_blocks(block, false))
+    if (!c->prompt_path || c->const_gain <= 0 || c->log_fn || blocks < pf_min_blocks(block, false, false))
         return false;
     bool wide = false;
+    uint32_t corr = 0;  // launches with corrections
     for (uint32_t l = 0; l < layer_count; l++) {
         for (int m = 0; m < M_COUNT; m++) {
             const Matrix& mt = c->mat(l, m);
@@ -2467,8 +2473,10 @@ bool prompt_path_ok(llm_ctx* c, uint32_t n_prompt, uint32_t block, uint32_t laye
         }
         const Matrix &g = c->mat(l, M_GATE), &u = c->mat(l, M_UP);
         if (!(g.p12_ok && u.p12_ok) && !(g.mf && u.mf)) return false;
+        corr += c->mat(l, M_QKV).corr_any + c->mat(l, M_O).corr_any +
+                (g.corr_any || u.corr_any) + c->mat(l, M_DOWN).corr_any;
     }
-    return blocks >= pf_min_blocks(block, wide);
+    return blocks >= pf_min_blocks(block, corr > layer_count, wide);
 }
 
 // Places the buffers for p.rows rows from p.base on (nowhere while that is

@@ -153,6 +153,26 @@ def test_split_products(monkeypatch, spec, n, kind):
     _compare(monkeypatch, spec, kind, n, 4)
 
 
+@pytest.mark.parametrize("kind,n,block,layered", [
+    ("plain", 24, 8, False), ("plain", 25, 8, True), ("plain", 4, 1, False), ("plain", 5, 1, True),
+    ("one corrected", 25, 8, True), ("corrections", 32, 8, False), ("corrections", 33, 8, True),
+    ("corrections", 5, 1, False), ("corrections", 6, 1, True), ("wide", 40, 8, False),
+    ("wide", 41, 8, True), ("wide", 6, 1, False), ("wide", 7, 1, True)])
+def test_where_it_begins(monkeypatch, kind, n, block, layered):
+    """The blocks from which a prompt runs layer by layer: more where the weights need
+    corrections in most launches, or 16 bits, as each is where it becomes the faster way."""
+    import llm_accel
+    monkeypatch.setenv("LLM_ACCEL_PROMPT", "1")
+    model = Model(D64, "plain" if kind == "one corrected" else kind)
+    if kind == "one corrected":
+        model.weight(0, 6)[3, 5] = 3000
+    with llm_accel.Accelerator(accel_shape(D64)) as a:
+        a.load_model(model)
+        a.kernel_timing(True)
+        a.generate(model.emb, list(range(n)), block, D64.layers, 0)
+        assert a.kernel_stats()["rope"][0] == (D64.layers if layered else 0)
+
+
 def test_prompts_that_outgrow_the_workspace(monkeypatch):
     """One context, prompts of growing and falling length: each is the first work on a
     workspace that has just been allocated, or runs in a larger one."""
