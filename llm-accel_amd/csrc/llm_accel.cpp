@@ -2544,7 +2544,8 @@ int run_prompt_layers(llm_ctx* c, const int16_t* rows_host, uint32_t n, uint32_t
                       uint32_t layer_count) {
     hipStream_t st = c->stream;
     auto& p = c->pf;
-    const uint32_t chunk = std::min(n, std::min(p.rows, kPfMaxRows) / block * block);
+    // whole blocks, unless it is all
+    const uint32_t cap = std::min(p.rows, kPfMaxRows), chunk = n <= cap ? n : cap / block * block;
     auto gemm = [&](const int8_t* x, uint32_t m, const Matrix& w, const Matrix* w2, int epi,
                     const int16_t* res, int16_t* out, int8_t* xp, const int16_t* gamma) -> int {
         llm::PfGemmArgs a{};
@@ -2789,8 +2790,7 @@ int llm_generate(llm_ctx_t* c, const int16_t* embedding, uint32_t vocab,
         HIP_TRY(hipEventRecord(ev_p0, c->stream));
         const bool layers = prompt_path_ok(c, n_prompt, block_size, layer_count);
         if (layers)
-            if (int r = prompt_buffers(c, std::min(n_prompt, kPfMaxRows / block_size * block_size)))
-                return r;
+            if (int r = prompt_buffers(c, std::min(n_prompt, kPfMaxRows))) return r;
         if (layers && c->pf.rows) {
             if (int r = run_prompt_layers(c, c->stage, n_prompt, block_size, layer_count)) return r;
             const uint32_t blocks = (uint32_t)cdiv(n_prompt, block_size);

@@ -3,8 +3,9 @@ block-by-block prompt, bit for bit: sampled tokens, every K/V row, both hidden
 pairs and the report's counts, over row counts at the edges of the 32-row pieces,
 64-position tiles and 64- / 128-row workgroup tiles, ragged block sizes, head_dims
 that fill the matrix cores' operands and that do not, 12-bit weights with and
-without corrections, 16-bit weights, and saturating queries, keys and values; and
-once against the oracle's block by block replay."""
+without corrections, 16-bit weights, and saturating queries, keys and values; prompts
+that run in several parts; and once against the oracle's block by block replay.  Every
+comparison checks from the launch counts that the two requests took the two paths."""
 import sys
 
 import numpy as np
@@ -71,7 +72,10 @@ def _request(monkeypatch, spec, model, prompt, block, gen, layer_major):
         a.load_lm_head(model.emb)
         for pair in (0, 1):  # rows that no block writes stay what they were
             a.upload(pair, np.full((8, spec.hidden), 7 + pair, np.int16))
+        a.kernel_timing(True)
         toks, st = a.generate(model.emb, prompt, block, spec.layers, gen)
+        parts = a.kernel_stats()["rope"][0] / spec.layers  # a launch of this path only
+        a.kernel_timing(False)
         kv = [a.kv_read(layer, h, 0, len(prompt)) for layer in range(spec.layers)
               for h in range(spec.kv_heads)]
         pairs = [a.download(p, 8) for p in (0, 1)]
@@ -79,10 +83,10 @@ def _request(monkeypatch, spec, model, prompt, block, gen, layer_major):
         a.task(18, 0, 1, len(prompt), 1, 0)
         more = a.download(0, 8)
     counts = {k: v for k, v in st.items() if not k.endswith("ms")}
-    return toks, kv, pairs, more, counts
+    return toks, kv, pairs, more, counts, parts
 
 
-def _compare(monkeypatch, spec, kind, n, block, gen=1):
+def _compare(monkeypatch, spec, kind, n, block, gen=1, parts=1):
     model = Model(spec, kind)
     rng = np.random.default_rng(n)
     prompt = [int(t) for t in rng.integers(0, spec.vocab, size=n)]
@@ -98,12 +102,14 @@ def _compare(monkeypatch, spec, kind, n, block, gen=1):
             f"pair {p}: {np.argwhere(got[2][p] != want[2][p])[:3]}"
     assert np.array_equal(got[3], want[3])
     assert got[4] == want[4]
+    assert want[5] == 0 and got[5] == parts
 
 
 @pytest.mark.parametrize("n,block", [(4, 1), (5, 1), (31, 8), (33, 5), (64, 8), (65, 8), (127, 3),
                                      (129, 8), (200, 7)])
 def test_row_counts(monkeypatch, n, block):
-    _compare(monkeypatch, D64, "plain", n, block)
+    # four rows one by one stay in blocks
+    _compare(monkeypatch, D64, "plain", n, block, parts=0 if (n, block) == (4, 1) else 1)
 
 
 @pytest.mark.parametrize("spec", [D128, D48, D32, D16], ids=lambda s: s.name)
@@ -120,6 +126,25 @@ def test_weights_and_saturation(monkeypatch, spec, kind):
 
 def test_long_prompt(monkeypatch):
     _compare(monkeypatch, D128, "plain", 1100, 8)
+
+
+# Prompts of more rows than run at a time (2,048, or the multiple of the block below):
+# later parts read the earlier rows' K/V pages, share a page with them where the block
+# does not divide 64, and may be shorter than a block.
+LONG64 = workloads.ShapeSpec("long64", 512, 256, 688, 2, 4, 2, 4300, 0.25, 0.5)
+LONG128 = workloads.ShapeSpec("long128", 512, 512, 700, 1, 4, 2, 4300, 0.125, 0.3)
+LONG48 = workloads.ShapeSpec("long48", 512, 480, 700, 1, 10, 2, 4300, 0.125, 0.3)
+
+
+@pytest.mark.parametrize("spec,kind,n,block,parts", [
+    (LONG64, "plain", 2048, 8, 1), (LONG64, "plain", 2049, 8, 2), (LONG64, "saturating", 2056, 8, 2),
+    (LONG64, "plain", 2047, 5, 1), (LONG64, "plain", 2049, 5, 2),
+    (LONG64, "corrections", 2100, 5, 2), (LONG64, "wide", 2051, 7, 2),
+    (LONG64, "plain", 4200, 8, 3), (LONG128, "plain", 2100, 5, 2), (LONG128, "saturating", 4100, 3, 3),
+    (LONG128, "extreme", 2081, 7, 2), (LONG48, "plain", 2075, 6, 2), (LONG48, "saturating", 2300, 8, 2)],
+    ids=lambda v: getattr(v, "name", str(v)))
+def test_prompts_in_parts(monkeypatch, spec, kind, n, block, parts):
+    _compare(monkeypatch, spec, kind, n, block, gen=2, parts=parts)
 
 
 # Shapes whose products have more tiles than workgroups, which then take several in
