@@ -112,8 +112,9 @@ hipError_t launch_keys_out(unsigned long long* keys, unsigned long long* host_ke
                            uint32_t seq, hipStream_t st);
 // `rows` rows of `cols` int16 between device memory and pinned host memory,
 // or within device memory (addresses 16-byte aligned; row strides in
-// elements; cols and strides multiples of 8, or one row of any length).  With a flag (pinned), seq is stored there once every value
-// is visible to the host; count is a device word that is 0 between launches.
+// elements; cols and strides multiples of 8, or one row of any length).
+// With a flag (pinned), seq is stored there once every value is visible to
+// the host; count is a device word that is 0 between launches.
 hipError_t launch_io_rows(const int16_t* src, uint32_t ld_src, int16_t* dst, uint32_t ld_dst,
                           uint32_t cols, uint32_t rows, uint32_t* count, uint32_t* flag,
                           uint32_t seq, hipStream_t st);

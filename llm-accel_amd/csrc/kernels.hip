@@ -1053,9 +1053,9 @@ __global__ __launch_bounds__(256) void lm_argmax_kernel(const int16_t* __restric
 }
 
 // The same for blocks of 3-8 rows on the matrix cores: the VALU kernel's
-// products grow with the rows (8 rows of the 151,936 x 2,048 table: 400 us
-// against 116 for one, whose time is the table's bytes; here 120).  With w = 256 a + b
-// + 128 and x = 256 c + d + 128 (signed bytes),
+// products grow with the rows (8 rows of the 151,936 x 2,048 table: call
+// 415-421 us against 107-116 for one, whose time is the table's bytes; here
+// 127-135, the kernel 117 of them).  With w = 256 a + b + 128 and x = 256 c + d + 128 (signed bytes),
 //   sum w x = 65536 sum ac + 256 (sum ad + sum bc) + sum bd
 //             + 128 sum (256 a + b) + 128 sum x,
 // all sums exact in int32 (hidden <= 3840 here): the MFMA's columns are the
@@ -1234,9 +1234,11 @@ static hipError_t launch_lm_rt(const int16_t* w, uint32_t steps, uint32_t n,
 hipError_t launch_lm_argmax(const int16_t* w, uint32_t steps, uint32_t n,
                             const int16_t* x, uint32_t ldx, uint32_t rows, int L,
                             unsigned long long* keys, hipStream_t st) {
-    // From three rows on the matrix cores (call times at hidden 2048, 151,936
-    // rows: 3 rows 236 -> 135 us, 5 410 -> 135, 8 415 -> 134; one and two
-    // rows 122 and 128 us against 134).  Tables of fewer groups than 2,048
+    // From three rows on the matrix cores (call times, dot2 -> matrix cores:
+    // 151,936 x 2,048, 3 rows 236 -> 127-135 us, 8 415 -> 128-135; 151,936 x
+    // 896 98 -> 57, 157 -> 57; 16,384 x 896 35 -> 22, 39 -> 22; 8,192 x 256
+    // 25 -> 18, 26 -> 18.  One and two rows stay on dot2: 106-109 and 118-120,
+    // 65 and 61, 17 and 18, 15 and 15).  Tables of fewer groups than 2,048
     // wavefronts can walk share each among a workgroup's wavefronts, at most
     // 512 of them (their final atomics share a line: 30,000 rows of 2,048 in
     // 38 us, 49 with a workgroup per group); larger ones take one workgroup

@@ -252,9 +252,10 @@ __global__ __launch_bounds__(256) void op_flash_kernel(OpFlashArgs a) {
 // the running maximum is a maximum, so it needs no sequence -- the tile's
 // probabilities, sum and PV values, (3) the sequential rescale of sums and
 // values, one addition per tile except where the maximum rises.  The walk
-// above takes ~5 us per tile; these three launches 7.5, 6.4 and 4.6 us at 8
-// tiles and 128 query rows (48 -> 18 us), little more at 24 (125 -> ~20).  K and V are staged clamped in LDS, in
-// the pages' bank-paired order (attn_common.h).
+// above takes ~5 us per tile; these three launches 6.8, 6.0 and 4.4 us at 8
+// tiles (16 heads of 128, commands back to back: 43.2 -> 15.8 us; at 16 tiles
+// 83.9 -> 18.0).  K and V are staged clamped in LDS, in the pages' bank-paired
+// order (attn_common.h).
 // ---------------------------------------------------------------------
 struct OpTile {
     uint32_t t, h, tile, n;  // token, KV head, tile, positions of the token
@@ -490,7 +491,11 @@ hipError_t launch_op_flash(const OpFlashArgs& a, hipStream_t st) {
     if (a.kv_heads * a.tokens * a.group == 0 || a.head_dim == 0 || a.head_dim > 128 ||
         a.head_dim % 16 != 0 || a.pos0 + a.tokens > a.tiles * 64)
         return hipErrorInvalidValue;
-    // the three launches from the tiles whose walk takes as long (~5 us each)
+    // The three launches from three tiles on.  Commands back to back, walk
+    // and launches, us: 16 / 2 heads of 128, three tiles, 8 tokens 17.7 / 14.7
+    // and one 17.5 / 14.2, two tiles 12.5 the walk; 4 / 2 heads of 64 14.2 /
+    // 9.8 and 13.8 / 9.5, two tiles 10.1; 14 / 2 of 64 14.3 / 12.1, 8 / 8 of
+    // 128 17.6 / 11.5.
     const uint32_t nt = (a.pos0 + a.tokens + 63) / 64;
     if (nt >= 3 && a.group <= 16 && a.tokens <= 8) {
         const uint32_t grid = a.tokens * a.kv_heads * nt;

@@ -980,7 +980,7 @@ __device__ __forceinline__ void pf_attention_body(const PfAttnArgs& a, PfAttnSme
             *(uint32_t*)&ps[rt][0][lane_off] = plane_c(w0 + 0x00800080u, w1 + 0x00800080u);
             *(uint32_t*)&ps[rt][1][lane_off] = __builtin_amdgcn_perm(w1, w0, 0x06040200u);
             if (vf) {
-                // c(p) in [-1023, 0], as 256 h + l
+                // c(p) in [-1024, 0] (p = 16384 has (8 - 16384) >> 4), as 256 h + l
                 const uint32_t u0 = pack16(sat_corr(p[0]), sat_corr(p[1]));
                 const uint32_t u1 = pack16(sat_corr(p[2]), sat_corr(p[3]));
                 *(uint32_t*)&ps[rt][3][lane_off] = __builtin_amdgcn_perm(u1, u0, 0x06040200u);
@@ -1031,7 +1031,9 @@ __device__ __forceinline__ void pf_attention_body(const PfAttnArgs& a, PfAttnSme
                 }
 #pragma unroll
                 for (int s = 0; s < 4; s++) {
-                    // |sum| <= 2^31 - 2^16: exact in 32 bits
+                    // sums in [-2^31, 2^31 - 2^16] (64 products of at most 2^14
+                    // and -2048, or 2048 with its correction of -1024): exact
+                    // in 32 bits, and so with 8224 added
                     const uint32_t tot = ((((uint32_t)ac[s] << 8) + (uint32_t)x[s]) << 8) +
                                          (uint32_t)bd[s];
                     // rnd(rnd(tot, 6), 8) = floor((tot + 2^5 + 2^13) / 2^14)
